@@ -63,7 +63,7 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def class_bytes_per_sample(precision, rps=0.0, ang64=16, sorted64=16):
+def class_bytes_per_sample(precision, rps=0.0, ang64=16, sorted64=16, lines=1.0):
     """Algorithmic HBM bytes per TOD sample of each operator kernel class
     (reads + writes of its streams; the map gathers hit the caches).
     FP64: pixel int32, (cos, sin) 2psi as two doubles, complex FP64 pair
@@ -74,13 +74,18 @@ def class_bytes_per_sample(precision, rps=0.0, ang64=16, sorted64=16):
     sums per record, P^T reads a 4-byte index and the record.  ang64: bytes of
     the FP64 angle in the gather and record passes (8 as a 64-bit turn, 16 as
     a pair); sorted64: bytes of the sorted angle that the FP64 P^T over
-    samples reads (8 as a 64-bit turn, 16 as a pair)."""
+    samples reads (8 as a 64-bit turn, 16 as a pair).  lines < 1: detectors
+    share lines of sight, lines of them per filtered stream; a sample is then a
+    sample of a stream, pixels, angles and piece words are read once per line,
+    the row pass reads the sets' mixing weights too (under 1 byte a sample, left
+    out) and a record holds five sums."""
     fp64 = precision == "fp64"
     ang = ang64 if fp64 else 4
     w = 8 if fp64 else 4
     z = 8 if fp64 else 4
     if rps:
-        return [4 + ang + w, 2 * w, w + ang + 8 / 16 + 3 * z * rps, (4 + 3 * z) * rps]
+        ns = 5 if lines < 1 else 3
+        return [(4 + ang) * lines + w, 2 * w, w + (ang + 8 / 16) * lines + ns * z * rps, (4 + ns * z) * rps]
     return [4 + ang + w,   # gather + column FFT: pixel, angle in; pair buffer out
             2 * w,         # row FFT + filter: pair buffer in and out
             w + z,         # inverse column FFT: pair buffer in, z out
@@ -314,7 +319,7 @@ def run_solve(cfg, pin, precision, precond, deflate, weights, steps, warmup, max
                final_true_residual=true_res,
                time_to_solution_s=(t_end - t0) if converged else None,
                device_bytes=ctx.device_bytes(), ms_per_step=ms_per_step, kernel_times=kt,
-               run_records=ctx.run_records(), fp64_angle_bytes=ctx.fp64_angle_bytes(),
+               run_records=ctx.run_records(), streams=ctx.streams(), fp64_angle_bytes=ctx.fp64_angle_bytes(),
                fp64_sorted_angle_bytes=ctx.fp64_sorted_angle_bytes())
     if un is not None:
         out["learned_stats"] = lstats
@@ -434,25 +439,27 @@ def main():
     n_ops = max(kt[4][1], 1)
     avg_ms = tot_ms / n_ops
     nrec, runs_on = head["run_records"]
-    rps = nrec / ntot if runs_on else 0.0
+    nstr, nline = head["streams"]
+    nfilt = ntot * nstr // cfg.ndet  # samples of the filtered streams
+    rps = nrec / nfilt if runs_on else 0.0
     names = CLASS_NAMES_RUNS if runs_on else CLASS_NAMES
     cbs = class_bytes_per_sample("fp64", rps, head["fp64_angle_bytes"],
-                                 head["fp64_sorted_angle_bytes"] or 16)
-    alg = ntot * cbs[dom]  # algorithmic bytes of the dominant kernel class per operator application
+                                 head["fp64_sorted_angle_bytes"] or 16, nline / nstr if nstr < cfg.ndet else 1.0)
+    alg = nfilt * cbs[dom]  # algorithmic bytes of the dominant kernel class per operator application
     achieved = alg / (avg_ms * 1e-3)
     for k in range(4):
         if kt[k][1]:
             log(f"  {names[k]}: {kt[k][0] / n_ops:.3f} ms per operator ({kt[k][1]} launches, "
-                f"{ntot * cbs[k] / (kt[k][0] / n_ops * 1e-3) / 1e12:.2f} TB/s of algorithmic bytes)")
+                f"{nfilt * cbs[k] / (kt[k][0] / n_ops * 1e-3) / 1e12:.2f} TB/s of algorithmic bytes)")
     apply_ms = kt[4][0] / max(kt[4][1], 1)
     lens = cfg.seglen if uneven else [cfg.ns] * cfg.ndet
     npix = head["npix"]
 
     def b_alg(s):
-        # whole-operator algorithmic bytes: the per-(detector, sample) stream
+        # whole-operator algorithmic bytes: the stream of each line of sight
         # read once (int32 pixel + cos 2psi + sin 2psi), the per-detector
         # noise weights, ~12 map-vector passes of the CG in FP64
-        return ntot * (4 + 2 * s) + sum(L // 2 + 1 for L in lens) * s + 12 * 3 * npix * 8
+        return ntot // cfg.ndet * nline * (4 + 2 * s) + sum(L // 2 + 1 for L in lens) * s + 12 * 3 * npix * 8
 
     traffic, traffic_src = read_traffic(args.workload, "fp64", names[dom])
     tts = head["time_to_solution_s"]
@@ -486,7 +493,8 @@ def main():
         "operator_alg_bytes": b_alg(8),
         "operator_frac_hbm": b_alg(8) / (apply_ms * 1e-3) / HBM_PEAK,
         "device_bytes": head["device_bytes"],
-        "run_records": {"records": nrec, "per_sample": nrec / ntot, "used": runs_on},
+        "run_records": {"records": nrec, "per_sample": rps, "used": runs_on},
+        "streams": {"filtered": nstr, "lines_of_sight": nline, "detectors": cfg.ndet},
         "fp64_angle_bytes": head["fp64_angle_bytes"],
         "fp64_sorted_angle_bytes": head["fp64_sorted_angle_bytes"],
         "roofline": {"bound": "hbm", "kernel": names[dom], "achieved": achieved / 1e9,

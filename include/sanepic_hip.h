@@ -318,12 +318,20 @@ int sanepic_kernel_time(sanepic_ctx *ctx, int32_t which, double *ms,
 int sanepic_device_bytes(sanepic_ctx *ctx, int64_t *bytes);
 /* The run layout of P^T (no counterpart in the reference, whose do_PtNd
  * scatters sample by sample, sanepic.cc:2584-2611): *nrec = runs of
- * consecutive samples in one pixel (aligned 16-sample pieces split them),
+ * consecutive samples in one pixel (aligned 16-sample pieces split them; a
+ * line of sight shared by several detectors, sanepic_streams, counts once),
  * *active = 1 when the operator's inverse column pass sums each run into one
  * record and P^T sums records; 0 when it writes z and P^T sums samples (the
  * layout is off, or the current segment length / FFT split cannot use it).
  * SANEPIC_RUNS=0 at creation turns the layout off. */
 int sanepic_run_records(sanepic_ctx *ctx, int64_t *nrec, int32_t *active);
+/* What an operator application filters (no counterpart in the reference, which
+ * filters every detector, sanepic.cc:2390-2637): *streams timelines over
+ * *lines lines of sight.  Four or more detectors with the same focal-plane
+ * offsets are three streams behind one line of sight, mixed bin by bin with
+ * their noise weights; otherwise each detector is a stream and a line of its
+ * own (both counts are then ndet). */
+int sanepic_streams(sanepic_ctx *ctx, int32_t *streams, int32_t *lines);
 /* Bytes per sample of the FP64 operator's polarisation angle in its gather
  * and record passes (no counterpart in the reference, which recomputes
  * cos/sin 2psi inside its loops): 8 when 2psi is stored as a 64-bit fraction

@@ -31,7 +31,7 @@ ABI_FUNCTIONS = [
     "sanepic_solve_step", "sanepic_get_map", "sanepic_get_nvar", "sanepic_get_sumcross",
     "sanepic_true_residual", "sanepic_set_profiling", "sanepic_kernel_time",
     "sanepic_device_bytes",
-    "sanepic_run_records",
+    "sanepic_run_records", "sanepic_streams",
     "sanepic_fp64_angle_bytes", "sanepic_fp64_sorted_angle_bytes",
     "sanepic_unet_create", "sanepic_unet_destroy", "sanepic_unet_last_error",
     "sanepic_unet_nparams", "sanepic_unet_init", "sanepic_unet_get_params",
@@ -137,6 +137,7 @@ def lib():
             "sanepic_kernel_time": [P, ctypes.c_int32, d_p, i64p],
             "sanepic_device_bytes": [P, i64p],
             "sanepic_run_records": [P, i64p, ctypes.POINTER(ctypes.c_int32)],
+            "sanepic_streams": [P, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)],
             "sanepic_fp64_angle_bytes": [P, ctypes.POINTER(ctypes.c_int32)],
             "sanepic_fp64_sorted_angle_bytes": [P, ctypes.POINTER(ctypes.c_int32)],
             "sanepic_unet_create": [i64, ctypes.c_int32, ctypes.POINTER(P)],
@@ -640,6 +641,13 @@ class Context:
         self._chk(lib().sanepic_fp64_sorted_angle_bytes(self.h, ctypes.byref(b)),
                   "fp64_sorted_angle_bytes")
         return b.value
+
+    def streams(self):
+        """(streams, lines of sight) that an operator application filters:
+        detectors with equal offsets share a line of sight."""
+        n, m = ctypes.c_int32(), ctypes.c_int32()
+        self._chk(lib().sanepic_streams(self.h, ctypes.byref(n), ctypes.byref(m)), "streams")
+        return n.value, m.value
 
     def run_records(self):
         """(number of run records, whether the operator uses them)."""

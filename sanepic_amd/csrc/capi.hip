@@ -81,25 +81,6 @@ int ilog2(int64_t v) {
 }
 
 // ---------------------------------------------------------------- profiling
-struct ProfScope {
-  sanepic_ctx *c;
-  int cls;
-  hipEvent_t a = nullptr, b = nullptr;
-  ProfScope(sanepic_ctx *c_, int cls_) : c(c_), cls(cls_) {
-    if (c->prof) {
-      (void)hipEventCreate(&a);
-      (void)hipEventCreate(&b);
-      (void)hipEventRecord(a, c->st);
-    }
-  }
-  ~ProfScope() {
-    if (c->prof && a) {
-      (void)hipEventRecord(b, c->st);
-      c->evs.emplace_back(cls, a, b);
-    }
-  }
-};
-
 int prof_collect(sanepic_ctx *c) {
   if (c->evs.empty()) return 0;
   HIPCHK(c, hipStreamSynchronize(c->st));
@@ -173,6 +154,11 @@ int build_weights(sanepic_ctx *c) {
   ACHK(c, dalloc(c, c->wt, c->ndet * N));
   if (c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->wt32, c->ndet * N));
   LCHK(c, launch_build_weights(dspn, c->ndet, N, c->g.N1, c->g.N2, c->wt, c->wt32, c->st));
+  if (use_streams(c)) {
+    ACHK(c, dalloc(c, c->mix, 6 * (int64_t)c->nset * N));
+    if (c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->mix32, 6 * (int64_t)c->nset * N));
+    LCHK(c, launch_build_mix(dspn, c->d_sdet, c->d_sbeg, c->nset, N, c->g.N1, c->g.N2, c->mix, c->mix32, c->st));
+  }
   HIPCHK(c, hipStreamSynchronize(c->st));
   dfree_later(c, dspn, c->ndet * H);
   return 0;
@@ -295,6 +281,7 @@ int run_scatter(sanepic_ctx *c, const T *z, double *q, int mask, const T *rec) {
   s.it = rec ? c->ritems.items : c->items;
   s.perm = rec ? c->rperm : c->perm;
   s.rec = rec;
+  s.rec5 = rec && use_streams(c) ? 1 : 0;
   if constexpr (sizeof(T) == 8) {
     s.cs_sorted = c->cs_sorted;
     s.turn_sorted = (rec || c->nc != 3) ? nullptr : c->turn_sorted64;
@@ -340,6 +327,7 @@ int apply_filter(sanepic_ctx *c, const double *x, bool chi2, bool use64, int64_t
         LCHK(c, launch_map_slots(x, c->gsrc, c->pix_nested ? c->mpos : nullptr, c->map64, c->npix, c->st, c->nc));
       a.map = c->map64;
     }
+    if (runs && use_streams(c)) return run_streams<double>(c, a, chi2, nb);
     int src = SRC_GATHER;
     if (c->pregather) {
       ACHK(c, dalloc(c, c->px64, c->ntot));
@@ -361,6 +349,7 @@ int apply_filter(sanepic_ctx *c, const double *x, bool chi2, bool use64, int64_t
     a.rec = c->rec32;
     a.rmeta = c->rmeta;
     a.recv = c->run_loads32;
+    if (use_streams(c)) return run_streams<float>(c, a, false, nb);
   }
   int src = SRC_GATHER;
   if (c->pregather) {
@@ -569,6 +558,8 @@ int set_split(sanepic_ctx *c, int log2n1) {
   }
   dfree(c, c->wt, c->ndet * c->ns);
   dfree(c, c->wt32, c->ndet * c->ns);
+  dfree(c, c->mix, 6 * (int64_t)c->nset * c->ns);
+  dfree(c, c->mix32, 6 * (int64_t)c->nset * c->ns);
   return c->pixelized ? sorted_turns(c) : 0;  // a split without run records
 }
 
@@ -1141,9 +1132,11 @@ int sanepic_pixelize(sanepic_ctx *c, int64_t *npix_out, int64_t *n_deferred) {
   }
   trace_mark("pixelize: sorted angles");
   ACHK(c, build_items(c, ntot, c->items_nested && c->d_slot2pix != nullptr));
+  ACHK(c, find_streams(c));
   ACHK(c, build_runs(c));
   ACHK(c, sorted_turns(c));
-  if (!c->pin_owner) dfree_later(c, c->d_slot2pix, npix);  // a group keeps it for fetch_host_order
+  // a group keeps it for fetch_host_order, shared lines of sight until the set-up (drop_streams)
+  if (!c->pin_owner && !c->nstream) dfree_later(c, c->d_slot2pix, npix);
   HIPCHK(c, hipStreamSynchronize(c->st));
   if (c->pin_owner) flush_frees(c);  // a group: its temporaries serve the next group
   trace_mark("pixelize: done");
@@ -1520,6 +1513,7 @@ int setup_pointing(sanepic_ctx *c) {
     ACHK(c, dalloc(c, c->z32, ntot));
     ACHK(c, dalloc(c, c->map32, c->nc * npix));
   }
+  if (!c->pin_owner) dfree_later(c, c->d_slot2pix, npix);
   if (c->nested_map && !c->pix_nested) ACHK(c, nest_gather_map(c));
   if (!c->nested_map) {  // pixels stay in ring order (get_pixels)
     c->h_slot2pix.clear();

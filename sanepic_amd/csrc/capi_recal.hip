@@ -127,6 +127,10 @@ int sanepic_set_recalib(sanepic_ctx *c, int32_t on) {
   HIPCHK(c, hipMemcpy(c->gain32, c->h_gain32.data(), nblk * sizeof(float), hipMemcpyHostToDevice));
   // P x is scaled by the gains in the pre-gather pass
   c->pregather = true;
+  if (c->pixelized) {
+    ACHK(c, drop_streams(c));
+    ACHK(c, sorted_turns(c));
+  }
   return SANEPIC_OK;
 }
 

@@ -96,7 +96,10 @@ bool use_runs(const sanepic_ctx *c) {
 }
 
 int build_runs(sanepic_ctx *c) {
-  const int64_t ntot = c->ntot, npix = c->npix;
+  // shared lines of sight have one run layout for all of their detectors
+  const int32_t *pix = c->nstream ? c->line_pix : c->pix;
+  const int64_t ntot = c->nstream ? c->nline * c->nseg * c->ns : c->ntot, npix = c->npix;
+  const int64_t nsum = c->nstream ? 5 : 3;
   if (!c->runs || c->pin_owner || !c->sub.empty() || c->single || c->zsorted || c->nc != 3) return 0;
   if (c->ns % 16 != 0 || ntot <= 0 || ntot >= (int64_t)INT32_MAX || npix <= 0) return 0;
   const int64_t npiece = ntot / 16;
@@ -106,7 +109,7 @@ int build_runs(sanepic_ctx *c) {
   ACHK(c, dalloc(c, rbase, npiece));
   ACHK(c, dalloc(c, rcnt, npiece));
   ACHK(c, dalloc(c, c->rmeta, npiece));
-  hipLaunchKernelGGL(k_run_ends, dim3(nblk256(npiece)), dim3(256), 0, c->st, c->pix, npiece, rend, rcnt);
+  hipLaunchKernelGGL(k_run_ends, dim3(nblk256(npiece)), dim3(256), 0, c->st, pix, npiece, rend, rcnt);
   HIPCHK(c, hipGetLastError());
   {
     size_t tb = 0;
@@ -124,7 +127,7 @@ int build_runs(sanepic_ctx *c) {
   if (nrec >= ((int64_t)1 << 48)) return fail(c, SANEPIC_EINVAL, "too many runs for the record layout");
   hipLaunchKernelGGL(k_run_meta, dim3(nblk256(npiece)), dim3(256), 0, c->st, rbase, rend, npiece, c->rmeta);
   ACHK(c, dalloc(c, keys, nrec));
-  hipLaunchKernelGGL(k_run_keys, dim3(nblk256(ntot)), dim3(256), 0, c->st, c->pix, rend, rbase, ntot, keys);
+  hipLaunchKernelGGL(k_run_keys, dim3(nblk256(ntot)), dim3(256), 0, c->st, pix, rend, rbase, ntot, keys);
   HIPCHK(c, hipGetLastError());
   ACHK(c, sort_keys(c, keys, nrec, npix, c->rperm, &skeys));
   int64_t *roff = nullptr;
@@ -138,8 +141,13 @@ int build_runs(sanepic_ctx *c) {
   HIPCHK(c, hipMemcpyAsync(hrc.data(), rc, npix * sizeof(int32_t), hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   ACHK(c, make_items(c, nrec, c->items_nested && c->d_slot2pix != nullptr, rc, roff, hrc, c->ritems));
-  ACHK(c, dalloc(c, c->rec64, 3 * nrec));
-  if (c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->rec32, 3 * nrec));
+  ACHK(c, dalloc(c, c->rec64, nsum * nrec));
+  if (c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->rec32, nsum * nrec));
+  if (c->nstream) {  // a detector on its own never writes the last two sums of its records
+    LCHK(c, launch_fill(c->rec64, 0.0, nsum * nrec, c->st));
+    if (c->rec32) HIPCHK(c, hipMemsetAsync(c->rec32, 0, nsum * nrec * sizeof(float), c->st));
+    dfree_later(c, c->line_pix, ntot);
+  }
   HIPCHK(c, hipStreamSynchronize(c->st));
   dfree_later(c, rcnt, npiece);
   dfree_later(c, rbase, npiece);

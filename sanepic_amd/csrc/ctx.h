@@ -151,8 +151,18 @@ struct sanepic_ctx {
   uint64_t *rmeta = nullptr;         // [ntot / 16] first record << 16 | run-end bits of each piece
   int run_loads32 = 0, run_loads64 = 0;  // load batching of the record pass (OpArgs::recv)
   uint32_t *rperm = nullptr;         // [nrec] pixel-sorted entry -> record
-  double *rec64 = nullptr;           // [nrec][3] FP64 operator's records
-  float *rec32 = nullptr;            // [nrec][3] FP32 operator's records
+  double *rec64 = nullptr;           // [nrec][3] FP64 operator's records ([nrec][5] with streams)
+  float *rec32 = nullptr;            // the same of the FP32 operator
+  // Detectors that share a line of sight (capi_streams.hip): nstream streams
+  // over nline lines of sight, the first nset of them sets of three streams
+  int nstream = 0, nset = 0, nline = 0;
+  int64_t nsdet = 0;
+  SkyStream *d_streams = nullptr;    // [nstream]
+  SkyDet *d_sdet = nullptr;          // the sets' detectors, set b at [d_sbeg[b], d_sbeg[b + 1])
+  int32_t *d_sbeg = nullptr;
+  int32_t *line_pix = nullptr;       // [nline][nseg ns] pixels (while the run layout is built)
+  double *mix = nullptr;             // [nset][6][N] mixing weights in row layout
+  float *mix32 = nullptr;
   ItemSet ritems;                    // P^T items over records
   bool pt_xcd = false;               // P^T items in XCD-contiguous ranges (SANEPIC_PT_XCD)
   bool mono_fft = false;             // deflation: A e_I by a full operator application (SANEPIC_MONO_FFT)
@@ -394,6 +404,26 @@ inline void trace_mark(const char *what) {
   last = now;
 }
 
+// Times the launches of its scope (kernel class cls) while profiling is on.
+struct ProfScope {
+  sanepic_ctx *c;
+  int cls;
+  hipEvent_t a = nullptr, b = nullptr;
+  ProfScope(sanepic_ctx *c_, int cls_) : c(c_), cls(cls_) {
+    if (c->prof) {
+      (void)hipEventCreate(&a);
+      (void)hipEventCreate(&b);
+      (void)hipEventRecord(a, c->st);
+    }
+  }
+  ~ProfScope() {
+    if (c->prof && a) {
+      (void)hipEventRecord(b, c->st);
+      c->evs.emplace_back(cls, a, b);
+    }
+  }
+};
+
 // The context whose pinned staging buffer a call uses.
 inline sanepic_ctx *pin_ctx(sanepic_ctx *c) { return c->pin_owner ? c->pin_owner : c; }
 
@@ -443,6 +473,13 @@ int sort_keys(sanepic_ctx *c, const uint32_t *keys, int64_t n, int64_t nkey, uin
 // records (the layout exists and the inverse pass can write it).
 int build_runs(sanepic_ctx *c);
 bool use_runs(const sanepic_ctx *c);
+// Shared lines of sight (capi_streams.hip): found at pixelisation before the
+// run layout; whether an operator application filters streams; its three
+// passes (run records out).
+int find_streams(sanepic_ctx *c);
+int drop_streams(sanepic_ctx *c);
+bool use_streams(const sanepic_ctx *c);
+template <typename T> int run_streams(sanepic_ctx *c, OpArgs<T> a, bool chi2, int64_t *nb);
 // The FP32 operator's pixel-sorted angles where it cannot use the run records
 // (after pixelisation and after every change of the FFT split)
 int sorted_turns(sanepic_ctx *c);

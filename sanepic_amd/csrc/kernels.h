@@ -85,6 +85,26 @@ enum : int {
   ROW_SRC_WT = 32,  // input = weights themselves (noise autocorrelation)
 };
 
+// One filtered stream of a context whose detectors share lines of sight.
+// Detectors with the same focal-plane offsets cross the same pixels, and the
+// polarisation angle of detector d is the leading detector's plus a constant:
+//   P x = I + cos(delta_d) A + sin(delta_d) B,
+//   A = Q cos 2psi + U sin 2psi, B = U cos 2psi - Q sin 2psi
+// (2psi the leader's).  The noise filter is linear, so a set of four or more
+// such detectors is filtered as the three streams I, A, B, mixed bin by bin
+// with H_jk = sum_d W_d e_dj e_dk, e_d = (1, cos delta_d, sin delta_d).
+struct SkyStream {
+  int32_t det;     // detector whose pixels and angles the stream reads
+  int32_t set;     // line of sight: its runs' place in rmeta
+  int32_t parts;   // 1: I alone, 2: Q and U alone, 3: all (a detector on its own)
+  int32_t slot;    // first of the run record's five sums that the stream writes
+  uint64_t turn;   // added to the angle (64-bit turn): a quarter turn for B
+};
+struct SkyDet {    // a detector of a set: its index and (cos, sin) of delta_d
+  int32_t det, pad;
+  double c, s;
+};
+
 template <typename T>
 struct OpArgs {
   using V = typename std::conditional<sizeof(T) == 8, double2, float2>::type;
@@ -127,6 +147,13 @@ struct OpArgs {
   T *rec;                 // [nrec][3]
   const uint64_t *rmeta;  // [ntot / 16]
   int recv;               // load batching / occupancy of the record pass (N2 = 256): 0 default
+  // Shared lines of sight (launch_*_streams): nset sets of three streams come
+  // first, then the detectors on their own; buf holds [stream][pair of segments][N].
+  const SkyStream *vs;    // [nvs]
+  int nvs, nset;
+  const T *mix;           // [nset][6][N] H_00 H_01 H_02 H_11 H_12 H_22 in row layout
+  const SkyDet *sdet;     // the sets' detectors, set b at [sbeg[b], sbeg[b + 1]) (chi2)
+  const int32_t *sbeg;
 };
 
 template <typename T> int launch_col_fwd(const OpArgs<T> &a, int src, hipStream_t s);
@@ -135,6 +162,17 @@ template <typename T> int launch_col_fwd(const OpArgs<T> &a, int src, hipStream_
 template <typename T> int launch_gather_px(const OpArgs<T> &a, T *px, int64_t ntot, hipStream_t s);
 template <typename T> int launch_row(const OpArgs<T> &a, hipStream_t s, int64_t *nblocks);
 template <typename T> int launch_col_inv(const OpArgs<T> &a, hipStream_t s);
+// The three passes over the streams of shared lines of sight (power-of-two
+// four-step lengths with N2 <= 256); the last writes run records of five sums.
+template <typename T> int launch_col_fwd_streams(const OpArgs<T> &a, hipStream_t s);
+template <typename T> int launch_row_streams(const OpArgs<T> &a, hipStream_t s, int64_t *nblocks);
+template <typename T> int launch_col_inv_streams(const OpArgs<T> &a, hipStream_t s);
+// mix[b][6][N] of the nset sets from the half spectra spn[det][0..N/2]; mix32 may be null
+int launch_build_mix(const double *spn, const SkyDet *sdet, const int32_t *sbeg, int nset, int64_t N, int64_t N1,
+                     int64_t N2, double *mix, float *mix32, hipStream_t s);
+// flag[d] = 1 where detector d's pixels differ anywhere from detector lead[d]'s
+int launch_same_pixels(const int32_t *pix, int64_t spd, const int32_t *lead, int64_t ndet, int32_t *flag,
+                       hipStream_t s);
 template <typename T> int launch_single(const OpArgs<T> &a, int src, hipStream_t s, int64_t *nblocks);
 
 // Pixel-sorted reduction (P^T): items are (pixel, entry range) chunks of the
@@ -164,6 +202,7 @@ struct ScatterArgs {
   const T *z;             // [ntot] time-domain values (in sorted order when `sorted`)
   const T *rec;           // or, when set, [nrec][3] run records: entries are runs and perm maps
                           // a sorted entry to its record (no angles are read)
+  int rec5;               // records of five sums (shared lines of sight): I, then (Q, U) twice
   int sorted;             // z is stored pixel-sorted: entry j at z[j]
   int xcd;                // XCD-contiguous item ranges (neighbouring pixels share an L2)
   int lanes;              // lanes per item: 4, 8 or 16 (fewer for short items; 0 means 16)

@@ -171,6 +171,54 @@ __global__ __launch_bounds__(256) void k_scatter(ScatterArgs<T> a) {
   }
 }
 
+// P^T over the run records of shared lines of sight: five sums a run, I and
+// twice (Q, U), summed as k_scatter sums records.
+template <typename T, int L>
+__global__ __launch_bounds__(256) void k_scatter_rec5(ScatterArgs<T> a) {
+  const int grp = threadIdx.x / L, lane = threadIdx.x % L;
+  const int64_t item = logical_block(a.xcd) * (256 / L) + grp;
+  if (item >= a.it.n) return;
+  const int p = a.it.pix[item];
+  const int64_t e0 = a.it.beg[item];
+  const int n = a.it.len[item];
+  T s0 = 0, s1 = 0, s2 = 0;
+  int k = lane;
+  for (; k + 3 * L < n; k += 4 * L) {
+    const int64_t j = e0 + k;
+    uint32_t pp[4];
+    T r[4][5];
+#pragma unroll
+    for (int u = 0; u < 4; u++) pp[u] = a.perm[j + L * u];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int v = 0; v < 5; v++) r[u][v] = a.rec[5 * (int64_t)pp[u] + v];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      s0 += r[u][0];
+      s1 += r[u][1] + r[u][3];
+      s2 += r[u][2] + r[u][4];
+    }
+  }
+  for (; k < n; k += L) {
+    const T *r = a.rec + 5 * (int64_t)a.perm[e0 + k];
+    s0 += r[0];
+    s1 += r[1] + r[3];
+    s2 += r[2] + r[4];
+  }
+  s0 = red_lanes<L>(s0);
+  s1 = red_lanes<L>(s1);
+  s2 = red_lanes<L>(s2);
+  if (lane == 0) {
+    const int slot = a.it.slot[item];
+    double *q = slot < 0 ? a.q + 3 * (int64_t)p : a.partial + 3 * (int64_t)slot;
+    const bool off = slot < 0 && a.mask && a.cnt[p] < 2;  // the Q/U mask (split pixels: k_fix)
+    q[0] = s0;
+    q[1] = off ? 0.0 : (double)s1;
+    q[2] = off ? 0.0 : (double)s2;
+  }
+}
+
 template <int NV>
 __global__ __launch_bounds__(256) void k_fix(Items it, const double *partial, double *out,
                                              const int32_t *cnt, int mask, const int32_t *oidx,
@@ -602,7 +650,12 @@ template <typename T>
 int launch_scatter(const ScatterArgs<T> &a, hipStream_t s) {
   if (a.rec && a.nc == 4) return -2;  // run records hold three sums
   if (a.it.n > 0) {
-    if (a.nc == 4)  // leakage component: 16 lanes per item
+    if (a.rec && a.rec5 && (a.qidx || a.accumulate)) return -2;  // uniform contexts only
+    if (a.rec && a.rec5 && a.lanes == 16)
+      hipLaunchKernelGGL((k_scatter_rec5<T, 16>), dim3(nblk(a.it.n, 16)), dim3(256), 0, s, a);
+    else if (a.rec && a.rec5)
+      hipLaunchKernelGGL((k_scatter_rec5<T, 8>), dim3(nblk(a.it.n, 32)), dim3(256), 0, s, a);
+    else if (a.nc == 4)  // leakage component: 16 lanes per item
       hipLaunchKernelGGL((k_scatter<T, 16, true>), dim3(nblk(a.it.n, 16)), dim3(256), 0, s, a);
     else if (a.rec && a.lanes == 4)
       hipLaunchKernelGGL((k_scatter<T, 4, false, true>), dim3(nblk(a.it.n, 64)), dim3(256), 0, s, a);

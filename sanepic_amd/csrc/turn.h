@@ -23,9 +23,11 @@ __device__ __forceinline__ uint32_t turn_of(double c, double s) {
 // |x| <= pi/4; sin x and cos x are their Taylor series to x^9 and x^10
 // (truncation below 2e-9 there); the quarter turn is a rotation,
 // (cos, sin)(q pi/2 + x) = (c, s), (-s, c), (-c, -s), (s, -c) for q = 0..3.
-__device__ __forceinline__ float2 cs_of_turn(uint32_t u) {
-  const uint32_t q = (u + 0x20000000u) >> 30;
-  const int32_t f = (int32_t)(u - (q << 30));             // |f| <= 2^29
+// With add, of the angle plus the turn `add` (an even multiple).
+__device__ __forceinline__ float2 cs_of_turn(uint32_t u, uint32_t add = 0) {
+  const uint32_t w = u + add;
+  const uint32_t q = (w + 0x20000000u) >> 30;
+  const int32_t f = (int32_t)(w - (q << 30));             // |f| <= 2^29
   const float x = (float)f * 1.46291807926715968e-9f;     // 2 pi / 2^32
   const float x2 = x * x;
   const float s = x + x * x2 * (-1.66666667e-1f + x2 * (8.33333333e-3f + x2 * (-1.98412698e-4f + x2 * 2.75573192e-6f)));
@@ -99,10 +101,11 @@ __device__ __forceinline__ double2 cs_of_turn64(uint64_t u) {
 // cos(A + x) = cos A + (cos A (cos x - 1) - sin A sin x) and
 // sin(A + x) = sin A + (sin A (cos x - 1) + cos A sin x):
 // about 20 fewer vector instructions a sample, within ~2e-16 of
-// cs_of_turn64.
-__device__ __forceinline__ double2 cs_of_turn64_tab(uint64_t u, const double2 *tab) {
-  const uint32_t j = (uint32_t)((u + ((uint64_t)1 << 55)) >> 56);
-  const int64_t f = (int64_t)(u - ((uint64_t)j << 56));  // |f| <= 2^55
+// cs_of_turn64.  With add, of the angle plus the turn `add`.
+__device__ __forceinline__ double2 cs_of_turn64_tab(uint64_t u, const double2 *tab, uint64_t add = 0) {
+  const uint64_t w = u + add;
+  const uint32_t j = (uint32_t)((w + ((uint64_t)1 << 55)) >> 56);
+  const int64_t f = (int64_t)(w - ((uint64_t)j << 56));  // |f| <= 2^55
   const double x = (double)f * 3.4061215800865545e-19;  // 2 pi / 2^64
   const double x2 = x * x;
   const double s = fma(x * x2, fma(x2, 1.0 / 120, -1.0 / 6), x);
