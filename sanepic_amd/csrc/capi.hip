@@ -323,8 +323,10 @@ int apply_filter(sanepic_ctx *c, const double *x, bool chi2, bool use64, int64_t
     }
     if (c->pix_nested || c->gsrc) {
       ACHK(c, dalloc(c, c->map64, c->nc * c->npix));
-      if (!c->map_filled)
+      if (!c->map_filled) {
+        c->map_has_d = false;
         LCHK(c, launch_map_slots(x, c->gsrc, c->pix_nested ? c->mpos : nullptr, c->map64, c->npix, c->st, c->nc));
+      }
       a.map = c->map64;
     }
     if (runs && use_streams(c)) return run_streams<double>(c, a, chi2, nb);
@@ -338,11 +340,13 @@ int apply_filter(sanepic_ctx *c, const double *x, bool chi2, bool use64, int64_t
     }
     return run_filter<double>(c, a, src, mode, nb);
   }
-  if (c->pix_nested || c->gsrc) {
-    if (!c->map_filled)
+  if (!c->map_filled) {
+    c->map_has_d = false;
+    if (c->pix_nested || c->gsrc)
       LCHK(c, launch_map_slots(x, c->gsrc, c->pix_nested ? c->mpos : nullptr, c->map32, c->npix, c->st, c->nc));
-  } else
-    LCHK(c, launch_d2f(x, c->map32, c->nc * c->npix, c->st));
+    else
+      LCHK(c, launch_d2f(x, c->map32, c->nc * c->npix, c->st));
+  }
   OpArgs<float> a = op_args<float>(c);
   a.map = c->map32;
   if (runs) {
@@ -428,6 +432,12 @@ CGArgs cg_args(sanepic_ctx *c) {
   a.sc = c->sc;
   a.part = c->part;
   a.az = c->deflate ? c->az : nullptr;
+  a.hsc = c->h_sc;
+  if (c->sub.empty()) {  // the map that apply_filter gathers the operator's input from
+    a.slot = c->pix_nested ? c->mpos : nullptr;
+    if (c->cfg.precision == SANEPIC_MIXED) a.map32 = c->map32;
+    else if (c->pix_nested) a.map64 = c->map64;
+  }
   return a;
 }
 
@@ -479,14 +489,18 @@ namespace {
 // Only kernel launches, so it can be captured into a graph.
 int enqueue_iteration(sanepic_ctx *c, bool refresh) {
   CGArgs a = cg_args(c);
-  ACHK(c, apply_A(c, c->d, c->q, 1, false, false));
-  LCHK(c, cg_launch_alpha(a, c->st));
+  c->map_filled = c->map_has_d;
+  const int rc = apply_A(c, c->d, c->q, 1, false, false);
+  c->map_filled = false;
+  ACHK(c, rc);
+  LCHK(c, cg_launch_dot(a, c->st));
   LCHK(c, cg_launch_update(a, refresh ? 1 : 0, c->st));
   if (refresh) {
     ACHK(c, apply_A(c, c->x, c->q, 1, !c->refresh32, !c->refresh32));
     LCHK(c, cg_launch_refresh_r(a, c->st));
   }
   LCHK(c, cg_launch_dir(a, c->st));
+  c->map_has_d = c->sub.empty();
   return 0;
 }
 
@@ -739,6 +753,7 @@ void sanepic_destroy(sanepic_ctx *c) {
   release_pool(c);
   if (!c->borrowed) trace_mark("destroy: device memory freed");
   if (c->h_pin) (void)hipHostFree(c->h_pin);
+  if (c->h_sc) (void)hipHostFree(c->h_sc);
   if (c->st && !c->borrowed) (void)hipStreamDestroy(c->st);
   if (c->up_pt) (void)hipStreamDestroy(c->up_pt);
   for (hipStream_t s : c->up_tod)
@@ -1507,7 +1522,7 @@ int setup_pointing(sanepic_ctx *c) {
   ACHK(c, dalloc(c, c->M, 6 * npix));
   ACHK(c, dalloc(c, c->nvar, c->nc * npix));
   if (c->nc == 4) ACHK(c, dalloc(c, c->ML, npix));
-  ACHK(c, dalloc(c, c->part, 8 * 512));
+  ACHK(c, dalloc(c, c->part, kCGPart));
   if (c->cfg.precision == SANEPIC_MIXED) {
     if (!c->single) ACHK(c, dalloc(c, c->buf32, c->g.npairs * N));
     ACHK(c, dalloc(c, c->z32, ntot));
@@ -1718,6 +1733,8 @@ int sanepic_solve_begin(sanepic_ctx *c, const sanepic_solve_opts *opts, const do
   const bool learned = c->precond == SANEPIC_PRECOND_LEARNED;
   if (c->nc == 4 && c->precond != SANEPIC_PRECOND_DIAG)
     return fail(c, SANEPIC_EINVAL, "the leakage component is solved with the reference's diagonal preconditioner only");
+  if (!c->h_sc) HIPCHK(c, hipHostMalloc((void **)&c->h_sc, sizeof(CGScalars), hipHostMallocDefault));
+  c->map_has_d = false;
   drop_graphs(c);
   c->use_graph = opts && opts->graph && !learned;
   if (learned && !c->un) return fail(c, SANEPIC_EINVAL, "no network attached (sanepic_learn_attach)");
@@ -1769,6 +1786,7 @@ int sanepic_solve_begin(sanepic_ctx *c, const sanepic_solve_opts *opts, const do
   } else {
     CGArgs a = cg_args(c);
     LCHK(c, cg_launch_init(a, c->st));
+    c->map_has_d = c->sub.empty();
   }
   const double var00 = opts ? opts->var00 : 0.0;
   if (var00 > 0.0) {  // the recalibration loop's crit denominator (1377-1385)
@@ -1791,6 +1809,14 @@ int sanepic_solve_step(sanepic_ctx *c, sanepic_iter_info *info) {
     return fpcg_step(c, info);
   }
   const bool refresh = (c->iter % c->refresh) == 0;
+  // the last direction's kernel filled the gather map, unless an application
+  // to another map came between (outside a captured iteration)
+  if (!c->map_has_d && c->sub.empty()) {
+    const CGArgs a = cg_args(c);
+    if (a.map64) LCHK(c, launch_map_slots(c->d, nullptr, a.slot, a.map64, c->npix, c->st, c->nc));
+    else if (a.map32) LCHK(c, launch_map_slots(c->d, nullptr, a.slot, a.map32, c->npix, c->st, c->nc));
+    c->map_has_d = true;
+  }
   if (c->use_graph && !c->prof) {
     hipGraphExec_t &gx = c->gexec[refresh ? 1 : 0];
     if (!gx) {
@@ -1811,9 +1837,8 @@ int sanepic_solve_step(sanepic_ctx *c, sanepic_iter_info *info) {
   } else {
     ACHK(c, enqueue_iteration(c, refresh));
   }
-  CGScalars h{};
-  HIPCHK(c, hipMemcpyAsync(&h, c->sc, sizeof(h), hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
+  const CGScalars h = *c->h_sc;  // written by the iteration's last kernel
   if (info) {
     info->iter = c->iter;
     info->crit = h.var_n / h.var00;

@@ -654,13 +654,13 @@ int sanepic_learn_harvest(sanepic_ctx *c, const sanepic_harvest_opts *o, int64_t
         crit = info.crit;
       } else {
         ACHK(c, apply_A(c, c->d, c->q, 1, false, true));
-        LCHK(c, cg_launch_alpha(a, c->st));
+        const bool refresh = (k % 10) == 0;
+        LCHK(c, cg_launch_dot(a, c->st));
+        LCHK(c, cg_launch_update(a, refresh ? 1 : 0, c->st));
         if (store)
           LCHK(c, launch_step_store(c->d, c->sc, store, n3, c->st));
         else
           LCHK(c, launch_step_tail(c->d, c->sc, c->tail, n3, c->st));
-        const bool refresh = (k % 10) == 0;
-        LCHK(c, cg_launch_update(a, refresh ? 1 : 0, c->st));
         if (refresh) {
           ACHK(c, apply_A(c, c->x, c->q, 1, false, true));
           LCHK(c, cg_launch_refresh_r(a, c->st));

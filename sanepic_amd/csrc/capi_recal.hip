@@ -188,6 +188,7 @@ int sanepic_recal_sums(sanepic_ctx *c, const double *x, double *sums) {
   a.gain = nullptr;
   a.zpos = nullptr;
   a.map = c->rc_map;
+  c->map_has_d = false;
   if (c->pix_nested) {
     LCHK(c, launch_map_slots(c->rc_map, nullptr, c->mpos, c->map64, npix, c->st, c->nc));
     a.map = c->map64;

@@ -345,7 +345,7 @@ int group_setup(sanepic_ctx *c) {
   ACHK(c, dalloc(c, c->q, 3 * npix));
   ACHK(c, dalloc(c, c->M, 6 * npix));
   ACHK(c, dalloc(c, c->nvar, 3 * npix));
-  ACHK(c, dalloc(c, c->part, 8 * 512));
+  ACHK(c, dalloc(c, c->part, kCGPart));
   HIPCHK(c, hipStreamSynchronize(c->st));
   trace_mark("group setup: union sums");
   flush_frees(c);

@@ -7,6 +7,8 @@
 // fixed kernel sequence; every reduction runs over a fixed grid (RGRID blocks,
 // grid-stride) and the partials are summed by one block in a fixed order, so
 // results are bit-reproducible from run to run.
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace {
@@ -47,13 +49,35 @@ __device__ __forceinline__ void apply_m(const CGArgs &a, int64_t p, const double
   z[3] = a.nc == 4 ? a.ML[p] * r[3] : 0.0;
 }
 
-constexpr int NP = 8;  // partial slots per block
-
-__device__ __forceinline__ void store_part(double *part, const double (&acc)[5]) {
+// Partials: value k of block b at part[k RGRID + b].  q.d has the first
+// RGRID, the residual's sums the five times RGRID after it (part + RGRID).
+template <int NV>
+__device__ __forceinline__ void store_part(double *part, const double (&acc)[NV]) {
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int k = 0; k < NP; k++) part[NP * blockIdx.x + k] = k < 5 ? acc[k] : 0.0;
+    for (int k = 0; k < NV; k++) part[k * RGRID + blockIdx.x] = acc[k];
   }
+}
+
+// The sums of the n blocks' partials, in every thread of the block.
+template <int NV>
+__device__ __forceinline__ void sum_part(const double *part, int n, double (&v)[NV], double (&sh)[NV][RBS / 64]) {
+#pragma unroll
+  for (int k = 0; k < NV; k++) v[k] = 0.0;
+  for (int i = threadIdx.x; i < n; i += RBS) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] += part[k * RGRID + i];
+  }
+#pragma unroll
+  for (int k = 0; k < NV; k++) v[k] = wave_sum(v[k]);
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) sh[k][threadIdx.x >> 6] = v[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; k++) v[k] = (sh[k][0] + sh[k][1]) + (sh[k][2] + sh[k][3]);
+  __syncthreads();  // sh may be used again
 }
 
 __global__ __launch_bounds__(RBS) void k_mask(double *v, const int32_t *cnt, int64_t npix, int nc) {
@@ -84,7 +108,7 @@ __device__ __forceinline__ void resid_terms(const CGArgs &a, int64_t p, const do
 __global__ __launch_bounds__(RBS) void k_init(CGArgs a) {
   __shared__ double sh[5][RBS / 64];
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)RGRID * RBS) {
+  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)gridDim.x * RBS) {
     double r[4] = {0.0, 0.0, 0.0, 0.0};
     for (int c = 0; c < a.nc; c++) {
       r[c] = a.b[a.nc * p + c] - a.q[a.nc * p + c];
@@ -94,77 +118,70 @@ __global__ __launch_bounds__(RBS) void k_init(CGArgs a) {
     resid_terms(a, p, r, acc);
   }
   block_sums<5>(acc, sh);
-  store_part(a.part, acc);
+  store_part(a.part + RGRID, acc);
 }
 
-// Partials of u.v (slot 0), or with isum of the I components of v - u (slot 3)
+// Partials of u.v, or with isum of the I components of v - u
 __global__ __launch_bounds__(RBS) void k_dot(CGArgs a, const double *u, const double *v, int isum) {
-  __shared__ double sh[5][RBS / 64];
-  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  __shared__ double sh[1][RBS / 64];
+  double acc[1] = {0.0};
   if (isum) {  // sum of the I components of v - u
-    for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)RGRID * RBS)
-      acc[3] += v[a.nc * p] - (u ? u[a.nc * p] : 0.0);
+    for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)gridDim.x * RBS)
+      acc[0] += v[a.nc * p] - (u ? u[a.nc * p] : 0.0);
   } else {
-    for (int64_t i = (int64_t)blockIdx.x * RBS + threadIdx.x; i < a.nc * a.npix; i += (int64_t)RGRID * RBS)
+    for (int64_t i = (int64_t)blockIdx.x * RBS + threadIdx.x; i < a.nc * a.npix; i += (int64_t)gridDim.x * RBS)
       acc[0] += u[i] * v[i];
   }
-  block_sums<5>(acc, sh);
+  block_sums<1>(acc, sh);
   store_part(a.part, acc);
 }
 
-// Sum the partials in block order and update the scalars.
+// The sums of a start, by one block:
 //   what 0: start (r0 set): delta0, var0, var00, coarse coefficient
-//   what 1: alpha = delta_n / q.d
-//   what 2: new residual: delta, var, beta, coarse coefficient
 //   what 3: true residual |b - q|^2, |b|^2 into tmp[0..1]
 //   what 4: einv = 1 / (Z^T A Z) from the I-sum of AZ
 //   what 5: y0 = einv * Z^T (b - q): starting coarse correction into tmp[2]
-__global__ __launch_bounds__(RBS) void k_final(CGArgs a, int what) {
-  __shared__ double sh[5][RBS / 64];
-  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int i = threadIdx.x; i < RGRID; i += RBS) {
-#pragma unroll
-    for (int k = 0; k < 5; k++) acc[k] += a.part[NP * i + k];
-  }
-  block_sums<5>(acc, sh);
+__global__ __launch_bounds__(RBS) void k_final(CGArgs a, int what, int n) {
+  __shared__ double sh[5][RBS / 64], sd[1][RBS / 64];
+  double acc[5], dot[1];
+  if (what == 0 || what == 3) sum_part<5>(a.part + RGRID, n, acc, sh);
+  else sum_part<1>(a.part, n, dot, sd);
   if (threadIdx.x != 0) return;
   CGScalars *sc = a.sc;
-  if (what == 0 || what == 2) {
+  if (what == 0) {
     const double c = a.az ? sc->einv * (acc[3] - acc[4]) : 0.0;  // A-DEF2 coarse step
     const double delta = acc[0] + c * acc[3];
     sc->coarse = c;
-    if (what == 0) {
-      sc->delta_n = delta;
-      sc->delta0 = delta;
-      sc->var_n = acc[1];
-      sc->var0 = acc[1];
-      sc->var00 = acc[2];
-      sc->beta = 0.0;
-    } else {
-      sc->delta_o = sc->delta_n;
-      sc->delta_n = delta;
-      sc->var_n = acc[1];
-      sc->beta = sc->delta_n / sc->delta_o;
-    }
-  } else if (what == 1) {
-    sc->rtq = acc[0];
-    sc->alpha = sc->delta_n / acc[0];
+    sc->delta_n = delta;
+    sc->delta0 = delta;
+    sc->var_n = acc[1];
+    sc->var0 = acc[1];
+    sc->var00 = acc[2];
+    sc->beta = 0.0;
   } else if (what == 3) {
     sc->tmp[0] = acc[0];
     sc->tmp[1] = acc[1];
   } else if (what == 4) {
-    sc->einv = acc[3] != 0.0 ? 1.0 / acc[3] : 0.0;
+    sc->einv = dot[0] != 0.0 ? 1.0 / dot[0] : 0.0;
   } else if (what == 5) {
-    sc->tmp[2] = sc->einv * acc[3];
+    sc->tmp[2] = sc->einv * dot[0];
   }
 }
 
-// x += alpha d; unless refresh: r -= alpha q and the residual partials
-__global__ __launch_bounds__(RBS) void k_update(CGArgs a, int refresh) {
-  __shared__ double sh[5][RBS / 64];
-  const double alpha = a.sc->alpha;
+// alpha = delta_n / q.d; x += alpha d; unless refresh: r -= alpha q and the
+// residual partials
+__global__ __launch_bounds__(RBS) void k_update(CGArgs a, int refresh, int n) {
+  __shared__ double sh[5][RBS / 64], sd[1][RBS / 64];
+  double dot[1];
+  sum_part<1>(a.part, n, dot, sd);
+  const double delta = a.sc->delta_n, alpha = delta / dot[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    a.sc->rtq = dot[0];
+    a.sc->alpha = alpha;
+    a.sc->delta_o = delta;
+  }
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)RGRID * RBS) {
+  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)gridDim.x * RBS) {
     for (int c = 0; c < a.nc; c++) a.x[a.nc * p + c] += alpha * a.d[a.nc * p + c];
     if (!refresh) {
       double r[4] = {0.0, 0.0, 0.0, 0.0};
@@ -175,15 +192,16 @@ __global__ __launch_bounds__(RBS) void k_update(CGArgs a, int refresh) {
       resid_terms(a, p, r, acc);
     }
   }
+  if (refresh) return;  // k_refresh writes the residual partials
   block_sums<5>(acc, sh);
-  store_part(a.part, acc);
+  store_part(a.part + RGRID, acc);
 }
 
 // r = b - q (q = A x, masked) and the residual partials
 __global__ __launch_bounds__(RBS) void k_refresh(CGArgs a) {
   __shared__ double sh[5][RBS / 64];
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)RGRID * RBS) {
+  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)gridDim.x * RBS) {
     double r[4] = {0.0, 0.0, 0.0, 0.0};
     for (int c = 0; c < a.nc; c++) {
       r[c] = a.b[a.nc * p + c] - a.q[a.nc * p + c];
@@ -192,18 +210,57 @@ __global__ __launch_bounds__(RBS) void k_refresh(CGArgs a) {
     resid_terms(a, p, r, acc);
   }
   block_sums<5>(acc, sh);
-  store_part(a.part, acc);
+  store_part(a.part + RGRID, acc);
 }
 
-// d = M r + Z c + beta d  (first: d = M r + Z c)
-__global__ __launch_bounds__(RBS) void k_dir(CGArgs a, int first) {
-  const double beta = a.sc->beta, c0 = a.sc->coarse;
-  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)RGRID * RBS) {
+// delta, |r|^2, beta and the coarse coefficient of the new residual, then
+// d = M r + Z c + beta d (first: the start's scalars, d = M r + Z c), written
+// to the gather map as well where the operator gathers from one.  Block 0
+// leaves the scalars for the host in pinned memory.
+__global__ __launch_bounds__(RBS) void k_dir(CGArgs a, int first, int n) {
+  __shared__ double sh[5][RBS / 64];
+  CGScalars *sc = a.sc;
+  double beta = 0.0, c0;
+  if (first) {
+    c0 = sc->coarse;
+  } else {
+    double acc[5];
+    sum_part<5>(a.part + RGRID, n, acc, sh);
+    c0 = a.az ? sc->einv * (acc[3] - acc[4]) : 0.0;  // A-DEF2 coarse step
+    const double delta = acc[0] + c0 * acc[3];
+    beta = delta / sc->delta_o;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      sc->coarse = c0;
+      sc->delta_n = delta;
+      sc->var_n = acc[1];
+      sc->beta = beta;
+      if (a.hsc) {
+        a.hsc->delta_n = delta;
+        a.hsc->var_n = acc[1];
+        a.hsc->beta = beta;
+        a.hsc->alpha = sc->alpha;
+        a.hsc->chi2 = sc->chi2;
+        a.hsc->var00 = sc->var00;
+        a.hsc->delta0 = sc->delta0;
+      }
+    }
+  }
+  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)gridDim.x * RBS) {
     double r[4] = {0.0, 0.0, 0.0, 0.0}, z[4];
     for (int c = 0; c < a.nc; c++) r[c] = a.r[a.nc * p + c];
     apply_m(a, p, r, z);
     z[0] += c0;
-    for (int c = 0; c < a.nc; c++) a.d[a.nc * p + c] = first ? z[c] : z[c] + beta * a.d[a.nc * p + c];
+    for (int c = 0; c < a.nc; c++) {
+      if (!first) z[c] += beta * a.d[a.nc * p + c];
+      a.d[a.nc * p + c] = z[c];
+    }
+    if (a.map64 || a.map32) {
+      const int64_t m = a.nc * (int64_t)(a.slot ? a.slot[p] : p);
+      for (int c = 0; c < a.nc; c++) {
+        if (a.map64) a.map64[m + c] = z[c];
+        else a.map32[m + c] = (float)z[c];
+      }
+    }
   }
 }
 
@@ -211,19 +268,19 @@ __global__ __launch_bounds__(RBS) void k_dir(CGArgs a, int first) {
 __global__ __launch_bounds__(RBS) void k_resid(CGArgs a) {
   __shared__ double sh[5][RBS / 64];
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int64_t i = (int64_t)blockIdx.x * RBS + threadIdx.x; i < a.nc * a.npix; i += (int64_t)RGRID * RBS) {
+  for (int64_t i = (int64_t)blockIdx.x * RBS + threadIdx.x; i < a.nc * a.npix; i += (int64_t)gridDim.x * RBS) {
     const double e = a.b[i] - a.q[i];
     acc[0] += e * e;
     acc[1] += a.b[i] * a.b[i];
   }
   block_sums<5>(acc, sh);
-  store_part(a.part, acc);
+  store_part(a.part + RGRID, acc);
 }
 
 // x_I += tmp[2]; q += tmp[2] * AZ  (starting coarse correction)
 __global__ __launch_bounds__(RBS) void k_coarse_start(CGArgs a) {
   const double y = a.sc->tmp[2];
-  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)RGRID * RBS) {
+  for (int64_t p = (int64_t)blockIdx.x * RBS + threadIdx.x; p < a.npix; p += (int64_t)gridDim.x * RBS) {
     a.x[a.nc * p] += y;
     for (int c = 0; c < a.nc; c++) a.q[a.nc * p + c] += y * a.az[a.nc * p + c];
   }
@@ -261,39 +318,45 @@ int cg_launch_mask(double *v, const int32_t *cnt, int64_t npix, hipStream_t s, i
   return ok();
 }
 
+// Blocks of the map kernels: one pixel a thread up to RGRID blocks.
+static inline int rgrid(const CGArgs &a) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(RGRID, (a.npix + RBS - 1) / RBS));
+}
+
 int cg_launch_init(const CGArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(k_init, dim3(RGRID), dim3(RBS), 0, s, a);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 0);
-  hipLaunchKernelGGL(k_dir, dim3(RGRID), dim3(RBS), 0, s, a, 1);
+  const int n = rgrid(a);
+  hipLaunchKernelGGL(k_init, dim3(n), dim3(RBS), 0, s, a);
+  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 0, n);
+  hipLaunchKernelGGL(k_dir, dim3(n), dim3(RBS), 0, s, a, 1, n);
   return ok();
 }
 
-int cg_launch_alpha(const CGArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(k_dot, dim3(RGRID), dim3(RBS), 0, s, a, (const double *)a.q, (const double *)a.d, 0);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 1);
+int cg_launch_dot(const CGArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_dot, dim3(rgrid(a)), dim3(RBS), 0, s, a, (const double *)a.q, (const double *)a.d, 0);
   return ok();
 }
 
 int cg_launch_update(const CGArgs &a, int refresh, hipStream_t s) {
-  hipLaunchKernelGGL(k_update, dim3(RGRID), dim3(RBS), 0, s, a, refresh);
-  if (!refresh) hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 2);
+  const int n = rgrid(a);
+  hipLaunchKernelGGL(k_update, dim3(n), dim3(RBS), 0, s, a, refresh, n);
   return ok();
 }
 
 int cg_launch_refresh_r(const CGArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(k_refresh, dim3(RGRID), dim3(RBS), 0, s, a);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 2);
+  hipLaunchKernelGGL(k_refresh, dim3(rgrid(a)), dim3(RBS), 0, s, a);
   return ok();
 }
 
 int cg_launch_dir(const CGArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(k_dir, dim3(RGRID), dim3(RBS), 0, s, a, 0);
+  const int n = rgrid(a);
+  hipLaunchKernelGGL(k_dir, dim3(n), dim3(RBS), 0, s, a, 0, n);
   return ok();
 }
 
 int cg_launch_resid(const CGArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL(k_resid, dim3(RGRID), dim3(RBS), 0, s, a);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 3);
+  const int n = rgrid(a);
+  hipLaunchKernelGGL(k_resid, dim3(n), dim3(RBS), 0, s, a);
+  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 3, n);
   return ok();
 }
 
@@ -311,16 +374,18 @@ int cg_launch_det_const(double *z, const double *w, int64_t spd, int64_t ntot, h
 
 int cg_launch_coarse_setup(const CGArgs &a, hipStream_t s) {
   // einv from the I components of AZ
-  hipLaunchKernelGGL(k_dot, dim3(RGRID), dim3(RBS), 0, s, a, (const double *)nullptr, (const double *)a.az, 1);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 4);
+  const int n = rgrid(a);
+  hipLaunchKernelGGL(k_dot, dim3(n), dim3(RBS), 0, s, a, (const double *)nullptr, (const double *)a.az, 1);
+  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 4, n);
   return ok();
 }
 
 int cg_launch_coarse_start(const CGArgs &a, hipStream_t s) {
   // y0 = einv * sum_I (b - q); x += y0 e_I; q += y0 AZ
-  hipLaunchKernelGGL(k_dot, dim3(RGRID), dim3(RBS), 0, s, a, (const double *)a.q, (const double *)a.b, 1);
-  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 5);
-  hipLaunchKernelGGL(k_coarse_start, dim3(RGRID), dim3(RBS), 0, s, a);
+  const int n = rgrid(a);
+  hipLaunchKernelGGL(k_dot, dim3(n), dim3(RBS), 0, s, a, (const double *)a.q, (const double *)a.b, 1);
+  hipLaunchKernelGGL(k_final, dim3(1), dim3(RBS), 0, s, a, 5, n);
+  hipLaunchKernelGGL(k_coarse_start, dim3(n), dim3(RBS), 0, s, a);
   return ok();
 }
 

@@ -90,7 +90,8 @@ struct sanepic_ctx {
   double *map_all64 = nullptr;
   float *map_all32 = nullptr;
   int32_t *map_src = nullptr;
-  bool map_filled = false;           // a group: its map is already filled for this application
+  bool map_filled = false;           // the gather map is already filled for this application
+  bool map_has_d = false;            // the gather map holds the PCG's direction d (cg.hip k_dir)
   int64_t *off = nullptr;
   uint32_t *perm = nullptr;
   int32_t *it_pix = nullptr, *it_len = nullptr, *it_slot = nullptr, *sp_pix = nullptr,
@@ -113,6 +114,7 @@ struct sanepic_ctx {
   double *x = nullptr, *r = nullptr, *d = nullptr, *q = nullptr, *M = nullptr, *nvar = nullptr,
          *part = nullptr, *tmpblk = nullptr;
   CGScalars *sc = nullptr;
+  CGScalars *h_sc = nullptr;         // pinned: the scalars of the iteration just completed
   int *zero_flag = nullptr;
   int iter = 0, refresh = 10, precond = 0;
   int64_t chunk = 0;  // pairs per four-step chunk (0: all at once)

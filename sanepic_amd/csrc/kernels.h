@@ -306,16 +306,25 @@ struct CGArgs {
   const double *ML;       // [npix] the leakage component's diagonal entry (nc == 4)
   const int32_t *cnt;     // mask source
   CGScalars *sc;
-  double *part;           // [512][8] partials
+  double *part;           // [kCGPart] block partials
   const double *az;       // A e_I for the monopole deflation, or null
+  CGScalars *hsc;         // pinned host copy that each new direction fills, or null
+  // the operator's gather map, which each new direction is written to as well
+  // (pixel p at slot[p], or at p): one of the two, or neither
+  double *map64;
+  float *map32;
+  const int32_t *slot;
 };
+constexpr int64_t kCGPart = 8 * 512;  // q.d and five sums of up to 512 blocks (the flexible PCG's kernels take 8 a block)
+
 
 int cg_launch_mask(double *v, const int32_t *cnt, int64_t npix, hipStream_t s, int nc = 3);
 int cg_launch_init(const CGArgs &a, hipStream_t s);      // r = b - q; d = M r; delta, var, var00
-int cg_launch_alpha(const CGArgs &a, hipStream_t s);     // rtq = q.d ; alpha = delta_n / rtq
-int cg_launch_update(const CGArgs &a, int refresh, hipStream_t s);  // x += alpha d; r -= alpha q (or nothing)
+int cg_launch_dot(const CGArgs &a, hipStream_t s);       // partials of q.d
+// alpha = delta_n / q.d (its partials in a.part); x += alpha d; r -= alpha q (or nothing)
+int cg_launch_update(const CGArgs &a, int refresh, hipStream_t s);
 int cg_launch_refresh_r(const CGArgs &a, hipStream_t s); // r = b - q
-int cg_launch_dir(const CGArgs &a, hipStream_t s);       // d = M r + beta d
+int cg_launch_dir(const CGArgs &a, hipStream_t s);       // delta, beta; d = M r + beta d
 int cg_launch_resid(const CGArgs &a, hipStream_t s);     // tmp[0] = |b - q|^2 (q = A x masked), tmp[1] = |b|^2
 // Monopole deflation (two-level A-DEF2 with Z = e_I): coarse vector, the
 // scalar 1/(Z^T A Z) from AZ, and the starting correction x += y0 Z.
