@@ -736,6 +736,11 @@ void sanepic_destroy(sanepic_ctx *c) {
   if (c->st) (void)hipStreamSynchronize(c->st);
   for (sanepic_ctx *s : c->sub) sanepic_destroy(s);  // groups borrow this stream
   c->sub.clear();
+  for (int k = 0; k < sanepic_ctx::kQueues - 1; k++) {  // joined to c->st after every use
+    if (c->qst[k]) (void)hipStreamDestroy(c->qst[k]);
+    if (c->qjoin[k]) (void)hipEventDestroy(c->qjoin[k]);
+  }
+  if (c->qfork) (void)hipEventDestroy(c->qfork);
   if (c->un) {  // the network outlives the context: give it back its stream
     c->un->net.st = c->un->own;
     c->un->attached = nullptr;

@@ -83,6 +83,12 @@ struct sanepic_ctx {
   // Per-detector lengths: P^T runs once over the union of the groups' samples
   // (gbase[k]: group k's first sample; its z is the slice of z / z32 there)
   bool union_pt = false;
+  // ... and its groups' filters side by side: group k on queue gqueue[k], 0 the
+  // context's stream, 1.. the streams below, joined to it by events
+  static constexpr int kQueues = 4;
+  hipStream_t qst[kQueues - 1] = {};
+  hipEvent_t qfork = nullptr, qjoin[kQueues - 1] = {};
+  std::vector<int> gqueue;
   std::vector<int64_t> gbase;
   // ... and one gather-map fill: the groups' maps are slices of one buffer
   // (group k's at moff[k] pixels), map position i filled from row map_src[i] of x
