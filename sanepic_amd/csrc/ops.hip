@@ -317,6 +317,152 @@ __device__ __forceinline__ void run_record(const OpArgs<T> &a, uint64_t meta, in
   }
 }
 
+// Columns of P <= 256: the M sub-FFTs side by side.  Thread group j of M (one
+// wave, or two from P = 128 on, which keeps B >= 8 columns a row) transforms
+// the j-th sub-columns of B = 16 G / P columns, the 16 M G values pass through
+// the LDS (FP64: real parts, then imaginary parts), and every thread then makes
+// the radix-M DFT of up to 6 (M = 3) or 4 (M = 5) outputs v.  The kernels above
+// run the sub-FFTs one after the other in the same 256 threads and pass their
+// values through the buffer's rows in HBM: bound by latency, since P = 16 makes
+// 256-column blocks, a few dozen of them in small contexts (3 detectors x 5
+// segments of 5 x 2^13: 18 blocks).  Gather + column pass of 15 to 25 pairs
+// of 5 x 2^15 or 3 x 2^15: 67 -> 34 and 44 -> 30 us, inverse 42 -> 19 and 23 ->
+// 15 us; on a full chip (64 detectors, 2^24 samples each, lengths up to 10 x
+// 2^20) the columns of all groups 9.1 -> 7.9 ms and 5.4 -> 4.7 ms (FP64).
+template <int LOG2P, int M, int GROUP = (LOG2P <= 6 ? 64 : 128)>
+struct ColM {
+  static constexpr int P = 1 << LOG2P, TS = P / 16, G = GROUP, B = G / TS, NV = 16 * G;
+  static constexpr int NT = G * M, NI = (NV + NT - 1) / NT;
+  static constexpr int R = LdsSize<LOG2P, B>::value;  // a group's exchange region
+};
+
+template <typename T, int LOG2P, int M, int SRC>
+__global__ __launch_bounds__((LOG2P <= 6 ? 64 : 128) * M) void k_col_fwd_mw(OpArgs<T> a) {
+  using V = VT<T>;
+  using C = ColM<LOG2P, M>;
+  constexpr int P = C::P, TS = C::TS, B = C::B, G = C::G, NV = C::NV, NT = C::NT, NI = C::NI;
+  constexpr bool SPLIT = sizeof(LdsE<V>) != sizeof(V);
+  __shared__ LdsE<V> lds[M * C::R];
+  const int tid = threadIdx.x, j = __builtin_amdgcn_readfirstlane(tid / G), lane = tid % G, b = lane % B, t = lane / B;
+  const int64_t N1 = a.g.N1, ncb = N1 / B, lb = logical_block(a.xcd), pr = lb / ncb, n1 = (lb % ncb) * B + b;
+  int det;
+  int64_t ga, gb;
+  pair_info(a.g, pr, det, ga, gb);
+  const bool hb = gb >= 0;  // unconditional b loads, as in col_fwd_body
+  const int64_t gbb = hb ? gb : ga;
+  V v[16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int64_t s = n1 + N1 * (int64_t)(j + M * (t + TS * i));
+    const T xa = load_src<T, SRC>(a, ga + s);
+    const T xb = load_src<T, SRC>(a, gbb + s);
+    v[i] = mk<V>(xa, hb ? xb : (T)0);
+  }
+  fft_reg<V, -1, LOG2P, B>(v, t, lds + j * C::R + b, a.tw4096);
+  V y[NI][M];
+  __syncthreads();  // every group's last FFT reads are done
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) lds[j * NV + i * G + lane] = v[i].x;
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NI; n++)
+#pragma unroll
+      for (int k = 0; k < M; k++) y[n][k].x = n * NT + tid < NV ? lds[k * NV + n * NT + tid] : (T)0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; i++) lds[j * NV + i * G + lane] = v[i].y;
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NI; n++)
+#pragma unroll
+      for (int k = 0; k < M; k++) y[n][k].y = n * NT + tid < NV ? lds[k * NV + n * NT + tid] : (T)0;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; i++) lds[j * NV + i * G + lane] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NI; n++)
+#pragma unroll
+      for (int k = 0; k < M; k++) y[n][k] = n * NT + tid < NV ? lds[k * NV + n * NT + tid] : mk<V>((T)0, (T)0);
+  }
+  // output twiddle w_N^{n1 k2}, k2 = vv + P q: w_N^{n1 vv} times powers of w_N^{n1 P}, in FP64
+  V *out = a.buf + pr * a.g.N;
+  const int64_t m1 = (lb % ncb) * B + tid % B;
+  const double2 wp = twN<double2, -1>(a.twlo64, a.twhi64, m1 * P);
+#pragma unroll
+  for (int n = 0; n < NI; n++) {
+    if (n * NT + tid < NV) {
+      const int64_t vv = (n * NT + tid) / B;
+      const double2 w1 = twN<double2, -1>(a.twlo64, a.twhi64, vv * N1);  // w_N2^{k vv}: its powers
+      double2 wk = w1;
+#pragma unroll
+      for (int k = 1; k < M; k++) {
+        y[n][k] = cmul(y[n][k], mk<V>((T)wk.x, (T)wk.y));
+        wk = cmul(wk, w1);
+      }
+      V Y[M];
+      dft_m<V, M, -1>(y[n], Y);
+      double2 w = twN<double2, -1>(a.twlo64, a.twhi64, m1 * vv);
+#pragma unroll
+      for (int q = 0; q < M; q++) {
+        out[(vv + (int64_t)P * q) * N1 + m1] = cmul(Y[q], mk<V>((T)w.x, (T)w.y));
+        w = cmul(w, wp);
+      }
+    }
+  }
+}
+
+// The inverse: radix-M DFTs first, their values to the sub-FFTs' groups
+// through the LDS whole (80 KB for M = 5 in FP64; in two halves the outputs
+// waiting in registers took 256 of them), then a wave per sub-FFT.
+template <typename T, int LOG2P, int M>
+__global__ __launch_bounds__(64 * M) void k_col_inv_mw(OpArgs<T> a) {
+  using V = VT<T>;
+  using C = ColM<LOG2P, M, 64>;
+  constexpr int P = C::P, TS = C::TS, B = C::B, G = C::G, NV = C::NV, NT = C::NT, NI = C::NI;
+  constexpr int XV = (int)(M * C::R * sizeof(LdsE<V>) / sizeof(V));  // the FFTs' exchanges use it afterwards
+  __shared__ V xch[M * NV > XV ? M * NV : XV];
+  const int tid = threadIdx.x, j = __builtin_amdgcn_readfirstlane(tid / G), lane = tid % G, b = lane % B, t = lane / B;
+  const int64_t N1 = a.g.N1, ncb = N1 / B, lb = logical_block(a.xcd), pr = lb / ncb, c0 = (lb % ncb) * B;
+  int det;
+  int64_t ga, gb;
+  pair_info(a.g, pr, det, ga, gb);
+  const V *in = a.buf + pr * a.g.N + c0 + tid % B;
+#pragma unroll 2
+  for (int n = 0; n < NI; n++) {
+    const int at = n * NT + tid;
+    if (at < NV) {
+      const int64_t vv = at / B;
+      V y[M], Z[M];
+#pragma unroll
+      for (int q = 0; q < M; q++) y[q] = in[(vv + (int64_t)P * q) * N1];
+      dft_m<V, M, +1>(y, Z);
+      const double2 w1 = twN<double2, +1>(a.twlo64, a.twhi64, vv * N1);  // w_N2^{-k vv}: its powers
+      double2 wk = w1;
+      xch[at] = Z[0];
+#pragma unroll
+      for (int k = 1; k < M; k++) {
+        xch[k * NV + at] = cmul(Z[k], mk<V>((T)wk.x, (T)wk.y));
+        wk = cmul(wk, w1);
+      }
+    }
+  }
+  __syncthreads();
+  V v[16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) v[i] = xch[j * NV + i * G + lane];
+  LdsE<V> *lds = reinterpret_cast<LdsE<V> *>(xch);  // the FFT's exchanges start with a barrier
+  fft_reg<V, +1, LOG2P, B>(v, t, lds + j * C::R + b, a.tw4096);
+  const T sa = seg_gain(a, ga), sb = gb >= 0 ? seg_gain(a, gb) : (T)1;
+#pragma unroll
+  for (int s = 0; s < 16; s++) {
+    const int64_t idx = c0 + b + N1 * (int64_t)(j + M * (t + TS * s));
+    a.z[zslot(a, ga + idx)] = v[s].x * sa;
+    if (gb >= 0) a.z[zslot(a, gb + idx)] = v[s].y * sb;
+  }
+}
+
 // ---------------------------------------------------------------- column inv
 template <typename T, int LOG2N2>
 __device__ __forceinline__ void col_inv_body(const OpArgs<T> &a, int64_t lb, LdsE<VT<T>> *lds) {
@@ -538,10 +684,23 @@ int launch_col_fwd_m(const OpArgs<T> &a, int src, hipStream_t s) {
     if (src == SRC_PX) return launch1(k_col_fwd_m<T, L, M, SRC_PX>, nb, s, a);          \
     if constexpr (sizeof(T) == 8) return launch1(k_col_fwd_m<T, L, M, SRC_RNG>, nb, s, a); \
     return -2;
+#define CFW1(L, SRC) launch1(k_col_fwd_mw<T, L, M, SRC>, a.g.npairs * (a.g.N1 / ColM<L, M>::B), s, a, ColM<L, M>::NT)
+#define CFW(L)                                                                              \
+  case L:                                                                                   \
+    if constexpr (sizeof(T) == 8)                                                           \
+      if (src == SRC_GATHER && a.ang64 && a.nc == 3) return CFW1(L, SRC_GATHER_T64);        \
+    if (src == SRC_GATHER) return CFW1(L, SRC_GATHER);                                      \
+    if (src == SRC_TOD) return CFW1(L, SRC_TOD);                                            \
+    if (src == SRC_PX) return CFW1(L, SRC_PX);                                              \
+    if constexpr (sizeof(T) == 8) return CFW1(L, SRC_RNG);                                  \
+    return -2;
   switch (a.g.log2N2) {
-    CFM(4) CFM(5) CFM(6) CFM(7) CFM(8) CFM(9) CFM(10)
+    CFW(4) CFW(5) CFW(6) CFW(7) CFW(8)
+    CFM(9) CFM(10)
     default: return -2;
   }
+#undef CFW
+#undef CFW1
 #undef CFM
 }
 
@@ -551,11 +710,14 @@ int launch_col_inv_m(const OpArgs<T> &a, hipStream_t s) {
   const int64_t nb = a.g.npairs * (a.g.N1 / B);
 #define CIM(L) \
   case L: return launch1(k_col_inv_m<T, L, M>, nb, s, a);
+#define CIW(L) \
+  case L: return launch1(k_col_inv_mw<T, L, M>, a.g.npairs * (a.g.N1 / ColM<L, M, 64>::B), s, a, 64 * M);
   switch (a.g.log2N2) {
-    CIM(4) CIM(5) CIM(6) CIM(7) CIM(8) CIM(9) CIM(10)
+    CIW(4) CIW(5) CIW(6) CIW(7) CIM(8) CIM(9) CIM(10)
     default: return -2;
   }
 #undef CIM
+#undef CIW
 }
 
 template <typename T>

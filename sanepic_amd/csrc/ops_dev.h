@@ -266,10 +266,10 @@ __device__ __forceinline__ double row_shr(double v) {
 }
 
 template <typename K, typename A>
-int launch1(K kern, int64_t nblocks, hipStream_t s, const A &a) {
+int launch1(K kern, int64_t nblocks, hipStream_t s, const A &a, int threads = 256) {
   if (nblocks <= 0) return 0;
   if (nblocks > 0x7fffffffLL) return -1;
-  hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(threads), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
