@@ -600,7 +600,11 @@ const char *sanepic_last_error(const sanepic_ctx *ctx) {
   return ctx->err.c_str();
 }
 
-int sanepic_create(const sanepic_config *cfg, sanepic_ctx **out) {
+}  // extern "C"
+
+namespace sctx {
+// pointing: with boresight buffers of its own (a group reads its parent's)
+int create_context(const sanepic_config *cfg, sanepic_ctx **out, bool pointing) {
   g_create_error.clear();
   if (!cfg || !out) {
     g_create_error = "null argument";
@@ -717,9 +721,12 @@ int sanepic_create(const sanepic_config *cfg, sanepic_ctx **out) {
   c->pt_ok.assign(c->nseg, 0);
   c->tod_ok.assign((size_t)c->ndet * c->nseg, 0);
   c->dip_ok.assign((size_t)c->ndet * c->nseg, 0);
-  int rc = dalloc(c, c->ra, c->nseg * ns);
-  if (!rc) rc = dalloc(c, c->dec, c->nseg * ns);
-  if (!rc) rc = dalloc(c, c->psi, c->nseg * ns);
+  int rc = 0;
+  if (pointing) {
+    rc = dalloc(c, c->ra, c->nseg * ns);
+    if (!rc) rc = dalloc(c, c->dec, c->nseg * ns);
+    if (!rc) rc = dalloc(c, c->psi, c->nseg * ns);
+  }
   if (!rc) rc = dalloc(c, c->sc, 1);
   if (!rc) rc = dalloc(c, c->zero_flag, 1);
   if (rc) {
@@ -730,6 +737,11 @@ int sanepic_create(const sanepic_config *cfg, sanepic_ctx **out) {
   *out = c;
   return SANEPIC_OK;
 }
+}  // namespace sctx
+
+extern "C" {
+
+int sanepic_create(const sanepic_config *cfg, sanepic_ctx **out) { return create_context(cfg, out, true); }
 
 void sanepic_destroy(sanepic_ctx *c) {
   if (!c) return;
@@ -754,8 +766,8 @@ void sanepic_destroy(sanepic_ctx *c) {
   if (c->up_pt) (void)hipStreamSynchronize(c->up_pt);
   for (hipStream_t s : c->up_tod)
     if (s) (void)hipStreamSynchronize(s);
-  for (void *p : c->allocs) (void)hipFree(p);
-  release_pool(c);
+  for (void *p : c->allocs) dev_release(c, p);
+  c->arena.free_all();
   if (!c->borrowed) trace_mark("destroy: device memory freed");
   if (c->h_pin) (void)hipHostFree(c->h_pin);
   if (c->h_sc) (void)hipHostFree(c->h_sc);
@@ -1654,15 +1666,12 @@ int sanepic_get_rhs(sanepic_ctx *c, double *bout) {
 
 int sanepic_apply(sanepic_ctx *c, const double *xin, double *yout) {
   ACHK(c, check_ready(c, true));
-  double *xd = nullptr, *yd = nullptr;
-  ACHK(c, dalloc(c, xd, c->nc * c->npix));
-  ACHK(c, dalloc(c, yd, c->nc * c->npix));
-  int rc = to_inter(c, xin, xd);
-  if (!rc) rc = apply_A(c, xd, yd, 0, false, c->cfg.precision == SANEPIC_FP64);
-  if (!rc) rc = from_inter(c, yd, yout);
-  dfree(c, xd, c->nc * c->npix);
-  dfree(c, yd, c->nc * c->npix);
-  return rc;
+  // a caller iterates: the product's two maps stay with the context
+  ACHK(c, dalloc(c, c->apply_x, c->nc * c->npix));
+  ACHK(c, dalloc(c, c->apply_y, c->nc * c->npix));
+  ACHK(c, to_inter(c, xin, c->apply_x));
+  ACHK(c, apply_A(c, c->apply_x, c->apply_y, 0, false, c->cfg.precision == SANEPIC_FP64));
+  return from_inter(c, c->apply_y, yout);
 }
 
 int sanepic_apply_noalloc(sanepic_ctx *c, const double *xin, double *yout) {
@@ -1698,19 +1707,14 @@ int sanepic_apply_noalloc(sanepic_ctx *c, const double *xin, double *yout) {
 
 int sanepic_chi2(sanepic_ctx *c, const double *xin, double *chi2) {
   ACHK(c, check_ready(c, true));
-  double *xd = nullptr, *yd = nullptr;
-  ACHK(c, dalloc(c, xd, c->nc * c->npix));
-  ACHK(c, dalloc(c, yd, c->nc * c->npix));
-  int rc = to_inter(c, xin, xd);
-  if (!rc) rc = apply_A(c, xd, yd, 0, true, true);
+  ACHK(c, dalloc(c, c->apply_x, c->nc * c->npix));
+  ACHK(c, dalloc(c, c->apply_y, c->nc * c->npix));
+  ACHK(c, to_inter(c, xin, c->apply_x));
+  ACHK(c, apply_A(c, c->apply_x, c->apply_y, 0, true, true));
   CGScalars h{};
-  if (!rc) {
-    rc = d2h(c, &h, c->sc, sizeof(h));
-  }
-  dfree(c, xd, c->nc * c->npix);
-  dfree(c, yd, c->nc * c->npix);
-  if (!rc) *chi2 = h.chi2;
-  return rc;
+  ACHK(c, d2h(c, &h, c->sc, sizeof(h)));
+  *chi2 = h.chi2;
+  return SANEPIC_OK;
 }
 
 

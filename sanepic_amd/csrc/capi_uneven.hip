@@ -401,7 +401,6 @@ int group_setup(sanepic_ctx *c) {
   HIPCHK(c, hipStreamSynchronize(c->st));
   trace_mark("group setup: union sums");
   flush_frees(c);
-  release_pool(c);
   trace_mark("group setup: deferred frees");
   c->setup_done = true;
   return SANEPIC_OK;
@@ -463,7 +462,7 @@ int sanepic_create_uneven(const sanepic_uneven_config *cfg, sanepic_ctx **out) {
     sc.ns = glen[g];
     sc.nseg = cfg->nsamp / glen[g];
     sanepic_ctx *s = nullptr;
-    const int rc = sanepic_create(&sc, &s);
+    const int rc = create_context(&sc, &s, false);
     if (rc) {
       cleanup();
       return rc;
@@ -476,7 +475,7 @@ int sanepic_create_uneven(const sanepic_uneven_config *cfg, sanepic_ctx **out) {
   pc.nseg = 1;
   pc.ns = 16;
   sanepic_ctx *c = nullptr;
-  int rc = sanepic_create(&pc, &c);
+  int rc = create_context(&pc, &c, false);
   if (rc) {
     cleanup();
     return rc;
@@ -487,9 +486,6 @@ int sanepic_create_uneven(const sanepic_uneven_config *cfg, sanepic_ctx **out) {
   if (const char *e = getenv("SANEPIC_UNION_PT")) c->union_pt = atoi(e) != 0;
   // the parent keeps only what a group context does not: the timeline
   // pointing (read by every group in place), the solver and the union map
-  dfree(c, c->ra, 16);
-  dfree(c, c->dec, 16);
-  dfree(c, c->psi, 16);
   c->tl_len = cfg->nsamp;
   c->ns = 0;
   c->nseg = 0;
@@ -509,9 +505,6 @@ int sanepic_create_uneven(const sanepic_uneven_config *cfg, sanepic_ctx **out) {
   c->ntot = 0;
   for (size_t g = 0; g < subs.size(); g++) {
     sanepic_ctx *s = subs[g];
-    dfree(s, s->ra, s->nseg * s->ns);
-    dfree(s, s->dec, s->nseg * s->ns);
-    dfree(s, s->psi, s->nseg * s->ns);
     s->ra = c->ra;
     s->dec = c->dec;
     s->psi = c->psi;

@@ -7,6 +7,8 @@
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <iterator>
+#include <map>
 #include <string>
 #include <tuple>
 #include <unordered_map>
@@ -29,6 +31,79 @@ struct ItemSet {
   int64_t nslots = 0;
   double *partial = nullptr;  // [nslots][8]
   int lanes = 16;             // lanes per item
+};
+
+// Device buffers of a context cut out of a few slabs.  An allocation of a few
+// megabytes costs 70 to 330 us here and its release 160 to 250 us, whatever its
+// size (below 1 MB the runtime has its own slabs: 1 us each): a run of 4
+// detectors x 6 x 2^17 samples from host buffers to maps spent 7 of its 13 ms
+// on a hundred of them (8.1 ms with the slabs).  Blocks given back serve later requests of
+// the same context (best fit, neighbours merged); the slabs are freed with it.
+// One host thread per context, as everything here; blocks are given back only
+// once the work that reads them is done.
+struct Arena {
+  std::map<char *, int64_t> slabs, spare;        // address -> bytes
+  std::unordered_map<void *, int64_t> used;
+  static constexpr int64_t kAlign = 4096;
+
+  // from the spare blocks; null if none fits
+  void *take(int64_t bytes) {
+    const int64_t n = (bytes + kAlign - 1) / kAlign * kAlign;
+    auto best = spare.end();
+    for (auto it = spare.begin(); it != spare.end(); ++it)
+      if (it->second >= n && (best == spare.end() || it->second < best->second)) best = it;
+    if (best == spare.end()) return nullptr;
+    char *p = best->first;
+    const int64_t rest = best->second - n;
+    spare.erase(best);
+    if (rest > 0) spare[p + n] = rest;
+    used[p] = n;
+    return p;
+  }
+  // a new slab of at least `bytes` (want: the size to try first)
+  hipError_t grow(int64_t bytes, int64_t want) {
+    void *v = nullptr;
+    int64_t n = (std::max(bytes, want) + kAlign - 1) / kAlign * kAlign;
+    hipError_t e = hipMalloc(&v, (size_t)n);
+    if (e != hipSuccess && want > bytes) {
+      (void)hipGetLastError();
+      n = (bytes + kAlign - 1) / kAlign * kAlign;
+      e = hipMalloc(&v, (size_t)n);
+    }
+    if (e != hipSuccess) return e;
+    slabs[(char *)v] = n;
+    spare[(char *)v] = n;
+    return hipSuccess;
+  }
+  // gives a block back; false if it is not the arena's
+  bool give(void *v) {
+    auto u = used.find(v);
+    if (u == used.end()) return false;
+    char *p = (char *)v;
+    int64_t n = u->second;
+    used.erase(u);
+    auto next = spare.lower_bound(p);
+    if (next != spare.begin()) {
+      auto prev = std::prev(next);
+      if (prev->first + prev->second == p && !slabs.count(p)) {  // blocks of two slabs stay apart
+        p = prev->first;
+        n += prev->second;
+        spare.erase(prev);
+      }
+    }
+    if (next != spare.end() && p + n == next->first && !slabs.count(next->first)) {
+      n += next->second;
+      spare.erase(next);
+    }
+    spare[p] = n;
+    return true;
+  }
+  void free_all() {
+    for (auto &s : slabs) (void)hipFree(s.first);
+    slabs.clear();
+    spare.clear();
+    used.clear();
+  }
 };
 
 struct sanepic_ctx {
@@ -140,11 +215,7 @@ struct sanepic_ctx {
   void *h_pin = nullptr;             // pinned host staging written by kernels (pixel counts)
   int64_t h_pin_bytes = 0;
   sanepic_ctx *pin_owner = nullptr;  // a group context stages through its parent's buffer
-  // A group's temporaries go back to its parent's pool when the group flushes
-  // them, and the next group's allocations take pool blocks first: the groups
-  // run one after another, so a few blocks serve all of them.
-  std::vector<std::pair<void *, int64_t>> pool;   // parent: free device blocks and their sizes
-  std::unordered_map<void *, int64_t> pool_cap;    // parent: size of every block its groups allocated
+  Arena arena;                       // this context's and its groups' device memory
   bool xcd_blocks = true;            // XCD-contiguous numbering of the four-step blocks
   bool zsorted = false;              // the filter output z is written in pixel-sorted order
   int col_waves = 3;                 // occupancy target of the FP32 gather column pass (0, 3, 4)
@@ -176,6 +247,7 @@ struct sanepic_ctx {
   bool mono_fft = false;             // deflation: A e_I by a full operator application (SANEPIC_MONO_FFT)
   double *px64 = nullptr;
   float *px32 = nullptr;
+  double *apply_x = nullptr, *apply_y = nullptr;  // [npix][nc] sanepic_apply's and sanepic_chi2's maps
   bool deflate = false;
   double *az = nullptr;
   bool begun = false, setup_done = false, pixelized = false;
@@ -266,34 +338,44 @@ int fail(sanepic_ctx *c, int code, const std::string &msg) {
 
 inline void flush_frees(sanepic_ctx *c);
 
+// The context that owns c's device memory: a group's parent.
+inline Arena &arena_of(sanepic_ctx *c) { return c->pin_owner ? c->pin_owner->arena : c->arena; }
+
+// Allocations of 1 MB up to kArenaMax come from the arena, a group's of any
+// larger size too: the groups' temporaries, released one group after the
+// other, serve the next group.
+constexpr int64_t kArenaMin = int64_t(1) << 20, kArenaMax = int64_t(1) << 27;
+
+inline hipError_t dev_alloc(sanepic_ctx *c, void **v, int64_t bytes) {
+  if (bytes < kArenaMin || (bytes >= kArenaMax && !c->pin_owner)) return hipMalloc(v, (size_t)bytes);
+  Arena &a = arena_of(c);
+  *v = a.take(bytes);
+  if (*v) return hipSuccess;
+  // a slab for a third of the context's per-sample state, 16 to 256 MB
+  const int64_t want = std::min<int64_t>(int64_t(1) << 28, std::max<int64_t>(int64_t(1) << 24, c->ntot * 32));
+  const hipError_t e = a.grow(bytes, want);
+  if (e == hipSuccess) *v = a.take(bytes);
+  return e;
+}
+
+// Releases device memory whose last reader has finished.
+inline void dev_release(sanepic_ctx *c, void *p) {
+  if (!arena_of(c).give(p)) (void)hipFree(p);
+}
+
 template <typename T>
 inline int dalloc(sanepic_ctx *c, T *&p, int64_t n) {
   if (p) return 0;
   if (n <= 0) n = 1;
   const int64_t bytes = (int64_t)((size_t)n * sizeof(T));
-  if (sanepic_ctx *o = c->pin_owner) {  // a group: the smallest pool block that fits, within 2x or 1 MB
-    size_t best = o->pool.size();
-    for (size_t i = 0; i < o->pool.size(); i++) {
-      const int64_t cap = o->pool[i].second;
-      if (cap >= bytes && cap <= std::max<int64_t>(2 * bytes, bytes + (1 << 20)) &&
-          (best == o->pool.size() || cap < o->pool[best].second))
-        best = i;
-    }
-    if (best < o->pool.size()) {
-      p = (T *)o->pool[best].first;
-      o->pool.erase(o->pool.begin() + (int64_t)best);
-      c->allocs.push_back((void *)p);
-      c->bytes += bytes;
-      return 0;
-    }
-  }
   void *v = nullptr;
-  hipError_t e = hipMalloc(&v, (size_t)n * sizeof(T));
+  hipError_t e = dev_alloc(c, &v, bytes);
   if (e != hipSuccess && !c->later.empty() && !c->pin_owner) {
     // set-up temporaries kept past the set-up (keep_temporaries) go first
     (void)hipGetLastError();
+    if (hipStreamSynchronize(c->st) != hipSuccess) (void)hipGetLastError();
     flush_frees(c);
-    e = hipMalloc(&v, (size_t)n * sizeof(T));
+    e = dev_alloc(c, &v, bytes);
   }
   if (e != hipSuccess) {
     (void)hipGetLastError();
@@ -304,18 +386,19 @@ inline int dalloc(sanepic_ctx *c, T *&p, int64_t n) {
   p = (T *)v;
   c->allocs.push_back(v);
   c->bytes += bytes;
-  if (c->pin_owner) c->pin_owner->pool_cap[v] = bytes;
   return 0;
 }
 
-// Frees a buffer this context allocated; a borrowed pointer is only dropped.
+// Frees a buffer this context allocated, after the work queued on its stream;
+// a borrowed pointer is only dropped.
 template <typename T>
 inline void dfree(sanepic_ctx *c, T *&p, int64_t n) {
   if (!p) return;
   auto it = std::find(c->allocs.begin(), c->allocs.end(), (void *)p);
   if (it != c->allocs.end()) {
     c->allocs.erase(it);
-    (void)hipFree(p);
+    if (c->st && hipStreamSynchronize(c->st) != hipSuccess) (void)hipGetLastError();
+    dev_release(c, (void *)p);
     c->bytes -= (int64_t)((size_t)std::max<int64_t>(n, 1) * sizeof(T));
   }
   p = nullptr;
@@ -337,12 +420,7 @@ inline void flush_frees(sanepic_ctx *c) {
     if (it == c->allocs.end()) continue;
     c->allocs.erase(it);
     c->bytes -= f.second;
-    sanepic_ctx *o = c->pin_owner;
-    auto cap = o ? o->pool_cap.find(f.first) : std::unordered_map<void *, int64_t>::iterator();
-    if (o && cap != o->pool_cap.end())
-      o->pool.emplace_back(f.first, cap->second);  // a group's temporary: back to the parent's pool
-    else
-      (void)hipFree(f.first);
+    dev_release(c, f.first);
   }
   c->later.clear();
 }
@@ -360,15 +438,6 @@ inline bool keep_temporaries(sanepic_ctx *c) {
     return false;
   }
   return (int64_t)fr >= (int64_t)(tot / 4);
-}
-
-// Frees the parent's pool of group temporaries.
-inline void release_pool(sanepic_ctx *c) {
-  for (auto &b : c->pool) {
-    c->pool_cap.erase(b.first);
-    (void)hipFree(b.first);
-  }
-  c->pool.clear();
 }
 
 // TOD upload stream k (mod kTodStreams), created on first use behind the
@@ -519,6 +588,7 @@ int group_pixelize(sanepic_ctx *c, int64_t *npix, int64_t *n_deferred);
 int group_setup(sanepic_ctx *c);
 // q = P^T N^-1 n (masked) for noise n with the detectors' spectra drawn from seed
 int noise_rhs(sanepic_ctx *c, uint64_t seed, double *q, int mask = 1);
+int create_context(const sanepic_config *cfg, sanepic_ctx **out, bool pointing);
 void set_create_error(const std::string &m);  // sanepic_last_error(NULL) of this thread
 // Flexible PCG with the attached network (capi_learn.hip): start after x0 and
 // the deflation set-up (q = A x0), and one iteration.
