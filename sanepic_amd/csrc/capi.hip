@@ -392,15 +392,56 @@ int check_ready(sanepic_ctx *c, bool need_setup) {
   return 0;
 }
 
+// Maps of up to 512 KB cross the bus inside the layout kernels, which read and
+// write pinned host memory: a copy of a few kilobytes from or to pageable
+// memory takes 12 to 20 us here, the kernels' own accesses 2 to 10 us (an
+// application to 6144 samples at NSIDE 16, with two such copies: 61 -> 47 us).
+// Larger maps go through the copy engines.  Every caller waits for its stream
+// before it returns, so one buffer serves both directions.
+constexpr int64_t kPinnedMap = int64_t(1) << 19;
+
+// The set-up's pinned buffers: the iteration's scalars and, if it is small, a map.
+int alloc_pinned(sanepic_ctx *c) {
+  const int64_t bytes = c->nc * c->npix * (int64_t)sizeof(double), head = 256;
+  static_assert(sizeof(CGScalars) <= 256, "scalars");
+  if (c->h_sc) return 0;
+  const bool map = bytes <= kPinnedMap;
+  HIPCHK(c, hipHostMalloc((void **)&c->h_sc, (size_t)(head + (map ? bytes : 0)), hipHostMallocDefault));
+  if (map) c->h_map = (double *)((char *)c->h_sc + head);
+  return 0;
+}
+
+static int pinned_map(sanepic_ctx *c, double **host, double **dev) {
+  *host = c->h_map;
+  *dev = nullptr;
+  if (c->h_map) HIPCHK(c, hipHostGetDevicePointer((void **)dev, c->h_map, 0));
+  return 0;
+}
+
 int to_inter(sanepic_ctx *c, const double *host_blk, double *dev_inter) {
-  ACHK(c, dalloc(c, c->tmpblk, c->nc * c->npix));
-  HIPCHK(c, hipMemcpyAsync(c->tmpblk, host_blk, c->nc * c->npix * sizeof(double), hipMemcpyHostToDevice,
-                           c->st));
-  LCHK(c, launch_block_to_inter(c->tmpblk, dev_inter, c->npix, c->st, c->nc));
+  double *host = nullptr, *dev = nullptr;
+  ACHK(c, pinned_map(c, &host, &dev));
+  if (host) {
+    std::memcpy(host, host_blk, (size_t)(c->nc * c->npix) * sizeof(double));
+  } else {
+    ACHK(c, dalloc(c, c->tmpblk, c->nc * c->npix));
+    HIPCHK(c, hipMemcpyAsync(c->tmpblk, host_blk, c->nc * c->npix * sizeof(double), hipMemcpyHostToDevice,
+                             c->st));
+    dev = c->tmpblk;
+  }
+  LCHK(c, launch_block_to_inter(dev, dev_inter, c->npix, c->st, c->nc));
   return 0;
 }
 
 int from_inter(sanepic_ctx *c, const double *dev_inter, double *host_blk) {
+  double *host = nullptr, *dev = nullptr;
+  ACHK(c, pinned_map(c, &host, &dev));
+  if (host) {
+    LCHK(c, launch_inter_to_block(dev_inter, dev, c->npix, c->st, c->nc));
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    std::memcpy(host_blk, host, (size_t)(c->nc * c->npix) * sizeof(double));
+    return 0;
+  }
   ACHK(c, dalloc(c, c->tmpblk, c->nc * c->npix));
   LCHK(c, launch_inter_to_block(dev_inter, c->tmpblk, c->npix, c->st, c->nc));
   HIPCHK(c, hipMemcpyAsync(host_blk, c->tmpblk, c->nc * c->npix * sizeof(double), hipMemcpyDeviceToHost,
@@ -1540,6 +1581,7 @@ int setup_pointing(sanepic_ctx *c) {
   ACHK(c, dalloc(c, c->nvar, c->nc * npix));
   if (c->nc == 4) ACHK(c, dalloc(c, c->ML, npix));
   ACHK(c, dalloc(c, c->part, kCGPart));
+  if (!c->pin_owner) ACHK(c, alloc_pinned(c));
   if (c->cfg.precision == SANEPIC_MIXED) {
     if (!c->single) ACHK(c, dalloc(c, c->buf32, c->g.npairs * N));
     ACHK(c, dalloc(c, c->z32, ntot));
@@ -1742,7 +1784,6 @@ int sanepic_solve_begin(sanepic_ctx *c, const sanepic_solve_opts *opts, const do
   const bool learned = c->precond == SANEPIC_PRECOND_LEARNED;
   if (c->nc == 4 && c->precond != SANEPIC_PRECOND_DIAG)
     return fail(c, SANEPIC_EINVAL, "the leakage component is solved with the reference's diagonal preconditioner only");
-  if (!c->h_sc) HIPCHK(c, hipHostMalloc((void **)&c->h_sc, sizeof(CGScalars), hipHostMallocDefault));
   c->map_has_d = false;
   drop_graphs(c);
   c->use_graph = opts && opts->graph && !learned;

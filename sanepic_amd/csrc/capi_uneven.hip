@@ -397,6 +397,7 @@ int group_setup(sanepic_ctx *c) {
   ACHK(c, dalloc(c, c->M, 6 * npix));
   ACHK(c, dalloc(c, c->nvar, 3 * npix));
   ACHK(c, dalloc(c, c->part, kCGPart));
+  ACHK(c, alloc_pinned(c));
   ACHK(c, make_queues(c));
   HIPCHK(c, hipStreamSynchronize(c->st));
   trace_mark("group setup: union sums");

@@ -195,6 +195,7 @@ struct sanepic_ctx {
   double *x = nullptr, *r = nullptr, *d = nullptr, *q = nullptr, *M = nullptr, *nvar = nullptr,
          *part = nullptr, *tmpblk = nullptr;
   CGScalars *sc = nullptr;
+  double *h_map = nullptr;           // pinned, behind h_sc: a small map on its way in or out, or null
   CGScalars *h_sc = nullptr;         // pinned: the scalars of the iteration just completed
   int *zero_flag = nullptr;
   int iter = 0, refresh = 10, precond = 0;
@@ -577,6 +578,7 @@ int apply_A(sanepic_ctx *c, const double *x, double *q, int mask, bool chi2, boo
 // (with runs: the records of the run layout instead of z)
 int apply_filter(sanepic_ctx *c, const double *x, bool chi2, bool use64, int64_t *nb, bool runs = false);
 int check_ready(sanepic_ctx *c, bool need_setup);
+int alloc_pinned(sanepic_ctx *c);
 int to_inter(sanepic_ctx *c, const double *host_blk, double *dev_inter);
 int from_inter(sanepic_ctx *c, const double *dev_inter, double *host_blk);
 int d2h(sanepic_ctx *c, void *dst, const void *src, size_t bytes);
