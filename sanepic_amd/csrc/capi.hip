@@ -1599,10 +1599,8 @@ int setup_pointing(sanepic_ctx *c) {
   // captures its first FP64 application, and no allocation may fall inside
   // a captured iteration
   if (c->pix_nested || c->pin_owner) ACHK(c, dalloc(c, c->map64, c->nc * npix));
-  if (c->pregather) {
-    ACHK(c, dalloc(c, c->px64, ntot));
-    if (c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->px32, ntot));
-  }
+  if (c->pregather || c->recal) ACHK(c, dalloc(c, c->px64, ntot));  // recal: the gain fit's model too
+  if (c->pregather && c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->px32, ntot));
   trace_mark("setup: pair sums, vectors (queued)");
   return 0;
 }

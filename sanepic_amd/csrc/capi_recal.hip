@@ -6,8 +6,8 @@
 //   * the NaN-filled TOD and the dipole stay resident after set-up, so b is
 //     rebuilt on the device for any gains: with x = d - g dip (one
 //     elementwise pass), b = P^T g N^-1 x, since g is one scalar per block;
-//   * the operator applies g twice per block: to P x in the pre-gather pass
-//     and to z in the inverse column pass (the context pre-gathers);
+//   * the operator applies g twice per block: to P x as it is gathered and to z
+//     in the inverse column pass;
 //   * the gain fit needs, per block, three half-spectrum sums
 //     H(u, v) = sum_{k <= ns/2} SpN_k Re(U_k conj V_k) of the reference's
 //     2185-2228 (U, V unnormalised r2c).  With z = c2r(SpN r2c v) -- the
@@ -142,8 +142,6 @@ int sanepic_set_recalib(sanepic_ctx *c, int32_t on) {
   ACHK(c, dalloc(c, c->gain32, nblk));
   HIPCHK(c, hipMemcpy(c->gain64, c->h_gain.data(), nblk * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(c->gain32, c->h_gain32.data(), nblk * sizeof(float), hipMemcpyHostToDevice));
-  // P x is scaled by the gains in the pre-gather pass
-  c->pregather = true;
   if (c->pixelized) {
     ACHK(c, drop_streams(c));
     ACHK(c, sorted_turns(c));

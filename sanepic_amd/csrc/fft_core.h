@@ -30,8 +30,11 @@ template <typename V> __device__ __forceinline__ V mk(decltype(V::x) a, decltype
 }
 template <typename V> __device__ __forceinline__ V cadd(V a, V b) { return mk<V>(a.x + b.x, a.y + b.y); }
 template <typename V> __device__ __forceinline__ V csub(V a, V b) { return mk<V>(a.x - b.x, a.y - b.y); }
+// explicit fused multiply-adds: which product of a sum the compiler fuses
+// depends on the code around it, and passes that read the same values from
+// different places must give the same bits
 template <typename V> __device__ __forceinline__ V cmul(V a, V b) {
-  return mk<V>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return mk<V>(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
 }
 template <typename V> __device__ __forceinline__ V cmulc(V a, V b) {  // a * conj(b)
   return mk<V>(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);

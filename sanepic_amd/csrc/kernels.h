@@ -134,7 +134,7 @@ struct OpArgs {
   int xcd;              // XCD-contiguous block numbering (four-step passes)
   int waves;            // occupancy target of the FP32 gather column pass (0: compiler's choice)
   const T *gain;        // [ndet][nseg] relative calibration of each segment, or null: it
-                        // multiplies P x in the pre-gather pass and z in the inverse pass
+                        // multiplies P x as it is gathered and z in the inverse pass
   int64_t blk;          // samples per (detector, segment) block (the block of sample g is g / blk)
   int rowdet;           // row pass: row k2 of all of a detector's pairs back to back (whole detectors only)
   // Runs: instead of z, the inverse column pass writes one record per run of

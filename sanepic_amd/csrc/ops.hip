@@ -76,6 +76,7 @@ __device__ __forceinline__ void col_fwd_body(const OpArgs<T> &a, int64_t lb, Lds
     const T xb = load_src<T, SRC, true>(a, gbb + s);
     v[i] = mk<V>(xa, hb ? xb : (T)0);
   }
+  gather_gain<T, SRC>(a, ga, gb, v);
   fft_reg<V, -1, LOG2N2, B>(v, t, lds + b, a.tw4096);
   V *out = a.buf + pr * a.g.N;
   TwRun tr = tw_run<-1>(a.twlo64, a.twhi64, n1 * t, n1 * TS);  // j = n1 k2, k2 = t + TS s
@@ -137,8 +138,8 @@ __device__ __forceinline__ void dft_m(const V (&y)[M], V (&Y)[M]) {
 #pragma unroll
     for (int j = 1; j < M; j++) {
       const int e = (j * q) % M;
-      acc.x += y[j].x * wr[e] - y[j].y * wi[e];
-      acc.y += y[j].x * wi[e] + y[j].y * wr[e];
+      acc.x = fma(y[j].x, wr[e], fma(-y[j].y, wi[e], acc.x));
+      acc.y = fma(y[j].x, wi[e], fma(y[j].y, wr[e], acc.y));
     }
     Y[q] = acc;
   }
@@ -174,6 +175,7 @@ __device__ __forceinline__ void col_fwd_m_body(const OpArgs<T> &a, int64_t lb, L
       const T xb = load_src<T, SRC>(a, gbb + s);
       v[i] = mk<V>(xa, hb ? xb : (T)0);
     }
+    gather_gain<T, SRC>(a, ga, gb, v);
     if (j) __syncthreads();  // the previous sub-FFT's last LDS reads
     fft_reg<V, -1, LOG2P, B>(v, t, lds + b, a.tw4096);
 #pragma unroll
@@ -358,6 +360,7 @@ __global__ __launch_bounds__((LOG2P <= 6 ? 64 : 128) * M) void k_col_fwd_mw(OpAr
     const T xb = load_src<T, SRC>(a, gbb + s);
     v[i] = mk<V>(xa, hb ? xb : (T)0);
   }
+  gather_gain<T, SRC>(a, ga, gb, v);
   fft_reg<V, -1, LOG2P, B>(v, t, lds + j * C::R + b, a.tw4096);
   V y[NI][M];
   __syncthreads();  // every group's last FFT reads are done
@@ -622,6 +625,7 @@ __global__ __launch_bounds__(256) void k_single(OpArgs<T> a) {
       const T xb = load_src<T, SRC>(a, gbb + s);
       v[i] = mk<V>(ha ? xa : (T)0, hb ? xb : (T)0);
     }
+    gather_gain<T, SRC>(a, gaa, gb, v);
   }
   double chi = 0.0;
   const int64_t base = pr * N;

@@ -30,9 +30,11 @@ __device__ __forceinline__ float2 cs_of_turn(uint32_t u, uint32_t add = 0) {
   const int32_t f = (int32_t)(w - (q << 30));             // |f| <= 2^29
   const float x = (float)f * 1.46291807926715968e-9f;     // 2 pi / 2^32
   const float x2 = x * x;
-  const float s = x + x * x2 * (-1.66666667e-1f + x2 * (8.33333333e-3f + x2 * (-1.98412698e-4f + x2 * 2.75573192e-6f)));
-  const float c = 1.0f + x2 * (-0.5f + x2 * (4.16666667e-2f + x2 * (-1.38888889e-3f +
-                                                                  x2 * (2.48015873e-5f - x2 * 2.75573192e-7f))));
+  // explicit fused multiply-adds: every kernel that decodes gets the same bits
+  const float s = fmaf(x * x2, fmaf(x2, fmaf(x2, fmaf(x2, 2.75573192e-6f, -1.98412698e-4f), 8.33333333e-3f),
+                                    -1.66666667e-1f), x);
+  const float c = fmaf(x2, fmaf(x2, fmaf(x2, fmaf(x2, fmaf(x2, -2.75573192e-7f, 2.48015873e-5f), -1.38888889e-3f),
+                                         4.16666667e-2f), -0.5f), 1.0f);
   float a = (q & 1) ? -s : c;
   float b = (q & 1) ? c : s;
   if (q & 2) {
