@@ -1568,6 +1568,7 @@ int setup_pointing(sanepic_ctx *c) {
   pa.nauto = c->nauto;
   pa.ns = c->ns;
   pa.nseg = c->nseg;
+  pa.ntot = ntot;
   pa.ns_shift = (c->ns & (c->ns - 1)) == 0 ? ilog2(c->ns) : -1;
   pa.out = c->pairs6;
   pa.partial = c->partial;

@@ -234,6 +234,7 @@ struct PairSumArgs {
   const int64_t *off;     // [npix+1] pixel offsets into the sorted list
   const double *nauto;    // [ndet][ns] c2r(|SpN|)
   int64_t ns, nseg;
+  int64_t ntot;           // entries of the sorted list
   int ns_shift;           // log2(ns) when ns is a power of two, else -1
   double *out;            // [npix][8]
   double *partial;        // [nslots][8]

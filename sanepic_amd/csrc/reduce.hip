@@ -276,9 +276,17 @@ __global__ __launch_bounds__(256) void k_crosslink(Items it, const double2 *cs, 
 // N^-1[t, t'] = nauto[(t - t') mod ns] and a = (1, cos 2psi, sin 2psi).
 // out[p][6]: the reference's I pair sum, which keeps only |t_j - t_k| < ns/2
 // (compute_diagPtNPCorr, sanepic.cc:2729-2752).
+//
+// Bound by the latency of a lane's chain (permutation, then the correlation at
+// the lag, four entries in flight): L lanes take an item, and the more lanes
+// there are the shorter is the chain and the more wavefronts hide it.  With 64
+// lanes instead of 16: 4.2 M samples of one detector on 22k pixels 4.6 -> 1.3 ms,
+// 3.1 M samples on 9k pixels 865 -> 338 us.  Filling a scan's last step of four
+// with zeros instead of single steps costs 10% at long groups.
+template <int L>
 __global__ __launch_bounds__(256) void k_pairsum(PairSumArgs a) {
-  const int grp = threadIdx.x >> 4, lane = threadIdx.x & 15;
-  const int64_t item = (int64_t)blockIdx.x * 16 + grp;
+  const int grp = threadIdx.x / L, lane = threadIdx.x % L;
+  const int64_t item = (int64_t)blockIdx.x * (256 / L) + grp;
   if (item >= a.it.n) return;
   const int p = a.it.pix[item];
   const int64_t e0 = a.it.beg[item];
@@ -294,7 +302,7 @@ __global__ __launch_bounds__(256) void k_pairsum(PairSumArgs a) {
   // the later entries k > j of its group once, with the off-diagonal terms
   // doubled: w (a_j a_k^T + a_k a_j^T).  The forward scan issues its loads
   // four entries at a time.
-  for (int kk = lane; kk < n; kk += 16) {
+  for (int kk = lane; kk < n; kk += L) {
     const int64_t j = e0 + kk;
     const uint32_t g = a.perm[j];
     const uint32_t blk = block_of(g), t = g - blk * ns;
@@ -349,7 +357,7 @@ __global__ __launch_bounds__(256) void k_pairsum(PairSumArgs a) {
     acc[6] += (half > 0 ? w0 : 0.0) + 2.0 * ut;
   }
 #pragma unroll
-  for (int v = 0; v < 7; v++) acc[v] = red16(acc[v]);
+  for (int v = 0; v < 7; v++) acc[v] = red_lanes<L>(acc[v]);
   if (lane == 0) {
     const int slot = a.it.slot[item];
     double *o = slot < 0 ? a.out + 8 * (int64_t)p : a.partial + 8 * (int64_t)slot;
@@ -694,7 +702,12 @@ int launch_crosslink(const Items &it, const double2 *cs_sorted, double *out, dou
 }
 
 int launch_pairsum(const PairSumArgs &a, hipStream_t s) {
-  if (a.it.n > 0) hipLaunchKernelGGL(k_pairsum, dim3(nblk(a.it.n, 16)), dim3(256), 0, s, a);
+  if (a.it.n > 0) {
+    // the line: 64 lanes win from about 50 entries an item (614k samples: 36 us
+    // against 58) and lose below 36 (4.2 M samples: 237 us against 225)
+    if (a.ntot >= 48 * a.it.n) hipLaunchKernelGGL(k_pairsum<64>, dim3(nblk(a.it.n, 4)), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_pairsum<16>, dim3(nblk(a.it.n, 16)), dim3(256), 0, s, a);
+  }
   if (a.it.nsplit > 0)
     hipLaunchKernelGGL(k_fix<8>, dim3(nblk(a.it.nsplit)), dim3(256), 0, s, a.it, a.partial, a.out,
                        (const int32_t *)nullptr, 0, (const int32_t *)nullptr, 0);
