@@ -44,15 +44,21 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
 
 constexpr int TX = 16, TY = 8, HX = TX + 2, HY = TY + 2;
 
-enum { EPI_RELU = 0, EPI_HEAD = 1, EPI_DATA = 2 };
+enum { EPI_RELU = 0, EPI_HEAD = 1, EPI_DATA = 2, EPI_MASK = 3 };
 
 // out[f][y][x][co] = epi( bias[co] + sum_{t, ci} W[co][t][ci] in[f][y+dy_t][x+dx_t][ci] )
 // A block computes CT of the output channels (blockIdx.x holds the tile column
 // and the channel group): all of them where the faces have tiles enough to
 // fill the chip, 16 on the coarse levels (conv_launch).
+// EPI_MASK is the data gradient through the ReLU whose output is mask (of the
+// shape of out): zero where that output is.  In the epilogue, where the sums
+// are in registers: as a kernel of its own the mask took 2 to 5 us a layer and
+// a launch's gap, 8 of the 15 layers (forward and gradient together at nside
+// 64: 877 -> 856 us).
 template <int CIN, int COUT, int CT, int EPI>
 __global__ __launch_bounds__(256) void k_conv3(const uint16_t *__restrict__ in, const uint16_t *__restrict__ W,
-                                               const float *__restrict__ bias, void *__restrict__ out, int S) {
+                                               const float *__restrict__ bias, const uint16_t *__restrict__ mask,
+                                               void *__restrict__ out, int S) {
   constexpr int PS = CIN + 8;  // LDS pixel stride in bf16 (16-byte aligned, staggers banks)
   constexpr int KT = 9 * CIN;
   constexpr int NKS = (KT + 31) / 32;
@@ -115,8 +121,14 @@ __global__ __launch_bounds__(256) void k_conv3(const uint16_t *__restrict__ in, 
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         v[q] = acc[j][m][q];
-        if constexpr (EPI != EPI_DATA) v[q] += bias[co + q];
+        if constexpr (EPI == EPI_RELU || EPI == EPI_HEAD) v[q] += bias[co + q];
         if constexpr (EPI == EPI_RELU) v[q] = v[q] > 0.f ? v[q] : 0.f;
+      }
+      if constexpr (EPI == EPI_MASK) {
+        const uint2 y = *reinterpret_cast<const uint2 *>(mask + o + co);
+        const uint16_t yq[4] = {(uint16_t)y.x, (uint16_t)(y.x >> 16), (uint16_t)y.y, (uint16_t)(y.y >> 16)};
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = bf2f(yq[q]) > 0.f ? v[q] : 0.f;
       }
       if constexpr (EPI == EPI_HEAD) {
         *reinterpret_cast<float4 *>((float *)out + o + co) = make_float4(v[0], v[1], v[2], v[3]);
@@ -350,18 +362,6 @@ __global__ __launch_bounds__(256) void k_skip_bwd(const uint16_t *__restrict__ d
   *reinterpret_cast<uint4 *>(gS + p * Cs + c8 * 8) = pack8(a);
 }
 
-// g = g * relu'(Y), in place (n = number of 8-element vectors)
-__global__ __launch_bounds__(256) void k_relu_bwd(uint16_t *__restrict__ g, const uint16_t *__restrict__ Y, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  float gv[8], yv[8];
-  unpack8(reinterpret_cast<const uint4 *>(g)[i], gv);
-  unpack8(reinterpret_cast<const uint4 *>(Y)[i], yv);
-#pragma unroll
-  for (int e = 0; e < 8; e++) gv[e] = yv[e] > 0.f ? gv[e] : 0.f;
-  reinterpret_cast<uint4 *>(g)[i] = pack8(gv);
-}
-
 __global__ __launch_bounds__(256) void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
                                               float *__restrict__ v, int64_t n, float lr, float b1, float b2,
                                               float eps, float wd, float c1, float c2) {
@@ -422,7 +422,8 @@ inline int lerr() { return hipGetLastError() == hipSuccess ? 0 : -1; }
 
 // ------------------------------------------------------------ dispatch tables
 template <int CIN, int COUT, int EPI>
-int conv_launch(const uint16_t *in, const uint16_t *W, const float *bias, void *out, int S, hipStream_t s) {
+int conv_launch(const uint16_t *in, const uint16_t *W, const float *bias, const uint16_t *mask, void *out, int S,
+                hipStream_t s) {
   dim3 grid((unsigned)((S + TX - 1) / TX), (unsigned)((S + TY - 1) / TY), (unsigned)kFaces);
   // Below 512 tiles (two a CU) the blocks split the output channels: on the
   // 8 x 8 faces of the deepest level 12 blocks of 128 channels waited on each
@@ -430,18 +431,18 @@ int conv_launch(const uint16_t *in, const uint16_t *W, const float *bias, void *
   if constexpr (COUT > 16) {
     if ((int64_t)grid.x * grid.y * grid.z < 512) {
       grid.x *= COUT / 16;
-      hipLaunchKernelGGL((k_conv3<CIN, COUT, 16, EPI>), grid, dim3(256), 0, s, in, W, bias, out, S);
+      hipLaunchKernelGGL((k_conv3<CIN, COUT, 16, EPI>), grid, dim3(256), 0, s, in, W, bias, mask, out, S);
       return lerr();
     }
   }
-  hipLaunchKernelGGL((k_conv3<CIN, COUT, COUT, EPI>), grid, dim3(256), 0, s, in, W, bias, out, S);
+  hipLaunchKernelGGL((k_conv3<CIN, COUT, COUT, EPI>), grid, dim3(256), 0, s, in, W, bias, mask, out, S);
   return lerr();
 }
 
-int conv_fwd(int cin, int cout, int epi, const uint16_t *in, const uint16_t *W, const float *bias, void *out, int S,
-             hipStream_t s) {
+int conv_fwd(int cin, int cout, int epi, const uint16_t *in, const uint16_t *W, const float *bias,
+             const uint16_t *mask, void *out, int S, hipStream_t s) {
 #define CONV_CASE(CI, CO, E) \
-  if (cin == CI && cout == CO && epi == E) return conv_launch<CI, CO, E>(in, W, bias, out, S, s);
+  if (cin == CI && cout == CO && epi == E) return conv_launch<CI, CO, E>(in, W, bias, mask, out, S, s);
   // forward (ReLU)
   CONV_CASE(16, 16, EPI_RELU)
   CONV_CASE(16, 32, EPI_RELU)
@@ -454,14 +455,14 @@ int conv_fwd(int cin, int cout, int epi, const uint16_t *in, const uint16_t *W, 
   CONV_CASE(96, 32, EPI_RELU)
   CONV_CASE(48, 16, EPI_RELU)
   CONV_CASE(16, 16, EPI_HEAD)
-  // data gradients (transposed shapes)
-  CONV_CASE(16, 16, EPI_DATA)
+  // data gradients (transposed shapes): into a ReLU's output, else plain
+  CONV_CASE(16, 16, EPI_MASK)
+  CONV_CASE(32, 32, EPI_MASK)
+  CONV_CASE(64, 64, EPI_MASK)
+  CONV_CASE(128, 128, EPI_MASK)
   CONV_CASE(16, 48, EPI_DATA)
-  CONV_CASE(32, 32, EPI_DATA)
   CONV_CASE(32, 96, EPI_DATA)
-  CONV_CASE(64, 64, EPI_DATA)
   CONV_CASE(64, 192, EPI_DATA)
-  CONV_CASE(128, 128, EPI_DATA)
   CONV_CASE(128, 64, EPI_DATA)
   CONV_CASE(64, 32, EPI_DATA)
   CONV_CASE(32, 16, EPI_DATA)
@@ -640,7 +641,8 @@ int net_forward(Net &n) {
   const ConvSpec *cv = n.conv;
   hipStream_t s = n.st;
   auto conv = [&](int i, const uint16_t *in, void *out, int epi) {
-    return conv_fwd(cv[i].cin, cv[i].cout, epi, in, n.wb + n.woff[i], n.p + n.boff[i], out, n.S[cv[i].level], s);
+    return conv_fwd(cv[i].cin, cv[i].cout, epi, in, n.wb + n.woff[i], n.p + n.boff[i], nullptr, out, n.S[cv[i].level],
+                    s);
   };
   auto pool = [&](const uint16_t *Y, uint16_t *P, int lc, int C) {
     const int64_t cnt = n.npx[lc] * (C / 8);
@@ -688,14 +690,11 @@ int net_backward(Net &n) {
                        cv[i].cin, cv[i].cout, n.g + n.woff[i], n.g + n.boff[i]);
     return lerr();
   };
-  // data gradient of conv i: out (cin channels) from G (cout channels)
-  auto dx = [&](int i, const uint16_t *G, uint16_t *out) {
-    return conv_fwd(cv[i].cout, cv[i].cin, EPI_DATA, G, n.wtb + n.woff[i], nullptr, out, n.S[cv[i].level], s);
-  };
-  auto relu = [&](uint16_t *g, const uint16_t *Y, int l, int C) {
-    const int64_t cnt = n.npx[l] * C / 8;
-    hipLaunchKernelGGL(k_relu_bwd, dim3(nblk(cnt)), dim3(256), 0, s, g, Y, cnt);
-    return lerr();
+  // data gradient of conv i: out (cin channels) from G (cout channels),
+  // through the ReLU with output Y where conv i reads one
+  auto dx = [&](int i, const uint16_t *G, uint16_t *out, const uint16_t *Y = nullptr) {
+    return conv_fwd(cv[i].cout, cv[i].cin, Y ? EPI_MASK : EPI_DATA, G, n.wtb + n.woff[i], nullptr, Y, out,
+                    n.S[cv[i].level], s);
   };
   auto upbwd = [&](const uint16_t *dU, const uint16_t *Yc, uint16_t *gC, int lc, int Cc, int Cs) {
     const int64_t cnt = n.npx[lc] * (Cc / 8);
@@ -709,53 +708,45 @@ int net_backward(Net &n) {
   };
   // head and level-0 decoder
   NCHK(dw(14, n.Y[13], n.gO));
-  NCHK(dx(14, n.gO, n.A[0]));
-  NCHK(relu(n.A[0], n.Y[13], 0, 16));
+  NCHK(dx(14, n.gO, n.A[0], n.Y[13]));
   NCHK(dw(13, n.Y[12], n.A[0]));
-  NCHK(dx(13, n.A[0], n.B[0]));
-  NCHK(relu(n.B[0], n.Y[12], 0, 16));
+  NCHK(dx(13, n.A[0], n.B[0], n.Y[12]));
   NCHK(dw(12, n.U[0], n.B[0]));
   NCHK(dx(12, n.B[0], n.C[0]));
   // level-1 decoder
   NCHK(upbwd(n.C[0], n.Y[11], n.A[1], 1, 32, 16));
   NCHK(dw(11, n.Y[10], n.A[1]));
-  NCHK(dx(11, n.A[1], n.B[1]));
-  NCHK(relu(n.B[1], n.Y[10], 1, 32));
+  NCHK(dx(11, n.A[1], n.B[1], n.Y[10]));
   NCHK(dw(10, n.U[1], n.B[1]));
   NCHK(dx(10, n.B[1], n.C[1]));
   // level-2 decoder
   NCHK(upbwd(n.C[1], n.Y[9], n.A[2], 2, 64, 32));
   NCHK(dw(9, n.Y[8], n.A[2]));
-  NCHK(dx(9, n.A[2], n.B[2]));
-  NCHK(relu(n.B[2], n.Y[8], 2, 64));
+  NCHK(dx(9, n.A[2], n.B[2], n.Y[8]));
   NCHK(dw(8, n.U[2], n.B[2]));
   NCHK(dx(8, n.B[2], n.C[2]));
   // bottom
   NCHK(upbwd(n.C[2], n.Y[7], n.A[3], 3, 128, 64));
   NCHK(dw(7, n.Y[6], n.A[3]));
-  NCHK(dx(7, n.A[3], n.B[3]));
-  NCHK(relu(n.B[3], n.Y[6], 3, 128));
+  NCHK(dx(7, n.A[3], n.B[3], n.Y[6]));
   NCHK(dw(6, n.P[3], n.B[3]));
   NCHK(dx(6, n.B[3], n.D[3]));
   // level-2 encoder
   NCHK(skbwd(n.C[2], n.D[3], n.Y[5], n.A[2], 2, 128, 64));
   NCHK(dw(5, n.Y[4], n.A[2]));
-  NCHK(dx(5, n.A[2], n.B[2]));
-  NCHK(relu(n.B[2], n.Y[4], 2, 64));
+  NCHK(dx(5, n.A[2], n.B[2], n.Y[4]));
   NCHK(dw(4, n.P[2], n.B[2]));
   NCHK(dx(4, n.B[2], n.D[2]));
   // level-1 encoder
   NCHK(skbwd(n.C[1], n.D[2], n.Y[3], n.A[1], 1, 64, 32));
   NCHK(dw(3, n.Y[2], n.A[1]));
-  NCHK(dx(3, n.A[1], n.B[1]));
-  NCHK(relu(n.B[1], n.Y[2], 1, 32));
+  NCHK(dx(3, n.A[1], n.B[1], n.Y[2]));
   NCHK(dw(2, n.P[1], n.B[1]));
   NCHK(dx(2, n.B[1], n.D[1]));
   // level-0 encoder
   NCHK(skbwd(n.C[0], n.D[1], n.Y[1], n.A[0], 0, 32, 16));
   NCHK(dw(1, n.Y[0], n.A[0]));
-  NCHK(dx(1, n.A[0], n.B[0]));
-  NCHK(relu(n.B[0], n.Y[0], 0, 16));
+  NCHK(dx(1, n.A[0], n.B[0], n.Y[0]));
   NCHK(dw(0, n.X0, n.B[0]));
   return 0;
 }
