@@ -59,7 +59,6 @@ struct Net {
   uint16_t *gO = nullptr;            // [L0][16] head gradient
   uint16_t *A[kLevels] = {}, *B[kLevels] = {}, *C[3] = {}, *D[kLevels] = {};
   float *dwpart = nullptr, *dbpart = nullptr;
-  int64_t dwpart_n = 0, dbpart_n = 0;
 };
 
 int net_create(Net &n, int64_t nside, hipStream_t st);

@@ -141,6 +141,17 @@ __global__ __launch_bounds__(256) void k_conv3(const uint16_t *__restrict__ in, 
   }
 }
 
+// The weight gradients whose partials wait for their sums.
+struct DwEntry {
+  const float *part, *bpart;
+  float *gW, *gb;
+  int ngrp, cin, cout, block0;
+};
+struct DwList {
+  DwEntry e[kConvs];
+  int n;
+};
+
 // Weight gradient partials: part[grp][t][co][ci] = sum over the block's
 // pixels p of G[p][co] * X[p + offset_t][ci]; tap 4 (no offset) blocks also
 // write the bias partial bpart[grp][co] = sum_p G[p][co].
@@ -225,43 +236,46 @@ __global__ __launch_bounds__(256) void k_conv3_dw(const uint16_t *__restrict__ X
   if (t == 4 && threadIdx.x < COUT) bpart[grp * COUT + threadIdx.x] = bsum;
 }
 
-// gW[co][t][ci] = sum_grp part[grp][t][co][ci]; gb[co] = sum_grp bpart[grp][co].
+// gW[co][t][ci] = sum_grp part[grp][t][co][ci]; gb[co] = sum_grp bpart[grp][co],
+// for the convolutions of a list (their blocks back to back in the grid).
 // Bound by the latency of the partials' loads (up to 512 of them an entry):
 // 32 neighbouring entries a block, 8 threads an entry that each take every 8th
 // partial with eight loads in flight, then their sums in a fixed order.  One
 // thread an entry with one load after the other took 65 us a convolution at
-// nside 64, now 4.6 us (forward and gradient together 1.99 -> 1.04 ms).
-__global__ __launch_bounds__(256) void k_dw_reduce(const float *__restrict__ part, const float *__restrict__ bpart,
-                                                   int64_t ngrp, int cin, int cout, float *__restrict__ gW,
-                                                   float *__restrict__ gb) {
+// nside 64, now 4.6 us (forward and gradient together 1.99 -> 1.04 ms), and
+// one launch for all convolutions instead of one each 856 -> 827 us.
+__global__ __launch_bounds__(256) void k_dw_reduce(DwList l) {
   __shared__ float red[8][32];
-  const int64_t nw = (int64_t)9 * cout * cin;
+  int k = 0;
+  while (k + 1 < l.n && (int)blockIdx.x >= l.e[k + 1].block0) k++;
+  const DwEntry e = l.e[k];
+  const int64_t nw = (int64_t)9 * e.cout * e.cin;
   const int o = threadIdx.x & 31, sp = threadIdx.x >> 5;
-  const int64_t j = (int64_t)blockIdx.x * 32 + o;  // entry in the partials' order [t][co][ci], then the bias
+  const int64_t j = (int64_t)((int)blockIdx.x - e.block0) * 32 + o;  // in the partials' order [t][co][ci], then the bias
   float s = 0.f;
-  if (j < nw + cout) {
-    const float *src = j < nw ? part + j : bpart + (j - nw);
-    const int64_t st = j < nw ? nw : cout;
-    int64_t g = sp;
-    for (; g + 56 < ngrp; g += 64) {
+  if (j < nw + e.cout) {
+    const float *src = j < nw ? e.part + j : e.bpart + (j - nw);
+    const int64_t st = j < nw ? nw : e.cout;
+    int g = sp;
+    for (; g + 56 < e.ngrp; g += 64) {
       float v[8];
 #pragma unroll
       for (int u = 0; u < 8; u++) v[u] = src[(g + 8 * u) * st];
 #pragma unroll
       for (int u = 0; u < 8; u++) s += v[u];
     }
-    for (; g < ngrp; g += 8) s += src[g * st];
+    for (; g < e.ngrp; g += 8) s += src[g * st];
   }
   red[sp][o] = s;
   __syncthreads();
-  if (sp == 0 && j < nw + cout) {
+  if (sp == 0 && j < nw + e.cout) {
 #pragma unroll
     for (int u = 1; u < 8; u++) s += red[u][o];
     if (j < nw) {
-      const int t = (int)(j / ((int64_t)cout * cin)), r = (int)(j % ((int64_t)cout * cin));
-      gW[((int64_t)(r / cin) * 9 + t) * cin + r % cin] = s;
+      const int t = (int)(j / ((int64_t)e.cout * e.cin)), r = (int)(j % ((int64_t)e.cout * e.cin));
+      e.gW[((int64_t)(r / e.cin) * 9 + t) * e.cin + r % e.cin] = s;
     } else {
-      gb[j - nw] = s;
+      e.gb[j - nw] = s;
     }
   }
 }
@@ -470,6 +484,11 @@ int conv_fwd(int cin, int cout, int epi, const uint16_t *in, const uint16_t *W, 
   return -2;
 }
 
+// Floats of weight gradient partials that wait for a common sum (a larger
+// convolution's alone otherwise): 128 MB, all of them at nside 64, and half of
+// the 256 MB cache that they are read back from.
+constexpr int64_t kDwPending = (int64_t)1 << 25;
+
 int64_t dw_groups(int64_t npx) { return std::min<int64_t>(512, npx / 64); }
 
 int conv_dw(int cin, int cout, const uint16_t *X, const uint16_t *G, float *part, float *bpart, int S, int64_t npx,
@@ -537,7 +556,7 @@ int net_create(Net &n, int64_t nside, hipStream_t st) {
   const ConvSpec spec[kConvs] = {{16, 16, 0},  {16, 16, 0},   {16, 32, 1},  {32, 32, 1}, {32, 64, 2},
                                  {64, 64, 2},  {64, 128, 3},  {128, 128, 3}, {192, 64, 2}, {64, 64, 2},
                                  {96, 32, 1},  {32, 32, 1},   {48, 16, 0},  {16, 16, 0}, {16, 16, 0}};
-  int64_t off = 0, maxpart = 0, maxb = 0;
+  int64_t off = 0, maxpart = 0, allpart = 0, allb = 0;
   for (int i = 0; i < kConvs; i++) {
     n.conv[i] = spec[i];
     n.woff[i] = off;
@@ -546,7 +565,8 @@ int net_create(Net &n, int64_t nside, hipStream_t st) {
     off += spec[i].cout;
     const int64_t ng = dw_groups(n.npx[spec[i].level]);
     maxpart = std::max<int64_t>(maxpart, ng * 9 * spec[i].cin * spec[i].cout);
-    maxb = std::max<int64_t>(maxb, ng * spec[i].cout);
+    allpart += ng * 9 * spec[i].cin * spec[i].cout;
+    allb += ng * spec[i].cout;
   }
   n.nparam = off;
   NCHK(nalloc(n, n.p, off));
@@ -576,10 +596,8 @@ int net_create(Net &n, int64_t nside, hipStream_t st) {
   NCHK(nalloc(n, n.D[1], n.npx[1] * 16));
   NCHK(nalloc(n, n.D[2], n.npx[2] * 32));
   NCHK(nalloc(n, n.D[3], n.npx[3] * 64));
-  NCHK(nalloc(n, n.dwpart, maxpart));
-  NCHK(nalloc(n, n.dbpart, maxb));
-  n.dwpart_n = maxpart;
-  n.dbpart_n = maxb;
+  NCHK(nalloc(n, n.dwpart, std::max(maxpart, std::min(allpart, kDwPending))));
+  NCHK(nalloc(n, n.dbpart, allb));
   NCHK(hipMemsetAsync(n.m, 0, off * sizeof(float), st) != hipSuccess);
   NCHK(hipMemsetAsync(n.v, 0, off * sizeof(float), st) != hipSuccess);
   NCHK(hipMemsetAsync(n.g, 0, off * sizeof(float), st) != hipSuccess);
@@ -681,14 +699,30 @@ int net_forward(Net &n) {
 int net_backward(Net &n) {
   const ConvSpec *cv = n.conv;
   hipStream_t s = n.st;
-  // weight gradient of conv i from its input X and pre-activation gradient G
+  // weight gradient of conv i from its input X and pre-activation gradient G:
+  // partials now, their sums in one launch for all convolutions, or as soon as
+  // the next one's do not fit in the workspace
+  DwList wait{};
+  int64_t used = 0, usedb = 0;
+  int blocks = 0;
+  auto reduce = [&]() {
+    if (!wait.n) return 0;
+    hipLaunchKernelGGL(k_dw_reduce, dim3((unsigned)blocks), dim3(256), 0, s, wait);
+    wait.n = blocks = 0;
+    used = usedb = 0;
+    return lerr();
+  };
   auto dw = [&](int i, const uint16_t *X, const uint16_t *G) {
     const int l = cv[i].level;
-    if (conv_dw(cv[i].cin, cv[i].cout, X, G, n.dwpart, n.dbpart, n.S[l], n.npx[l], s)) return -1;
-    const int64_t cnt = (int64_t)9 * cv[i].cin * cv[i].cout + cv[i].cout;
-    hipLaunchKernelGGL(k_dw_reduce, dim3((unsigned)((cnt + 31) / 32)), dim3(256), 0, s, n.dwpart, n.dbpart, dw_groups(n.npx[l]),
-                       cv[i].cin, cv[i].cout, n.g + n.woff[i], n.g + n.boff[i]);
-    return lerr();
+    const int64_t ng = dw_groups(n.npx[l]), cnt = (int64_t)9 * cv[i].cin * cv[i].cout;
+    if (used + ng * cnt > kDwPending && reduce()) return -1;
+    float *part = n.dwpart + used, *bpart = n.dbpart + usedb;
+    if (conv_dw(cv[i].cin, cv[i].cout, X, G, part, bpart, n.S[l], n.npx[l], s)) return -1;
+    wait.e[wait.n++] = {part, bpart, n.g + n.woff[i], n.g + n.boff[i], (int)ng, cv[i].cin, cv[i].cout, blocks};
+    blocks += (int)((cnt + cv[i].cout + 31) / 32);
+    used += ng * cnt;
+    usedb += ng * cv[i].cout;
+    return 0;
   };
   // data gradient of conv i: out (cin channels) from G (cout channels),
   // through the ReLU with output Y where conv i reads one
@@ -748,6 +782,7 @@ int net_backward(Net &n) {
   NCHK(dw(1, n.Y[0], n.A[0]));
   NCHK(dx(1, n.A[0], n.B[0], n.Y[0]));
   NCHK(dw(0, n.X0, n.B[0]));
+  NCHK(reduce());
   return 0;
 }
 
