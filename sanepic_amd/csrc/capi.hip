@@ -1530,7 +1530,8 @@ int setup_pointing(sanepic_ctx *c) {
   ACHK(c, dalloc(c, c->z, ntot));
   ACHK(c, dalloc(c, c->dspec, c->g.npairs * N));
   if (!c->single) ACHK(c, dalloc(c, c->buf, c->g.npairs * N));
-  const int64_t nchi = c->single ? c->g.npairs : c->g.npairs * (N / 4096);
+  int64_t nchi = c->single ? c->g.npairs : c->g.npairs * (N / 4096);
+  if (c->nstream) nchi = std::max(nchi, stream_row_blocks(c->g, c->nstream, c->nset));
   ACHK(c, dalloc(c, c->chi2part, nchi + 1));
   c->nchi2 = nchi;
   ACHK(c, dalloc(c, c->b_raw, c->nc * npix));

@@ -165,6 +165,11 @@ template <typename T> int launch_col_inv(const OpArgs<T> &a, hipStream_t s);
 // The three passes over the streams of shared lines of sight (power-of-two
 // four-step lengths with N2 <= 256); the last writes run records of five sums.
 template <typename T> int launch_col_fwd_streams(const OpArgs<T> &a, hipStream_t s);
+// (the row pass has stream_row_blocks blocks, each with a chi2 partial)
+// Below this many pair values over all streams the passes are bound by latency
+// and launches, not by bandwidth.
+constexpr int64_t kStreamsSmall = int64_t(1) << 22;
+int64_t stream_row_blocks(const PairGeom &g, int nvs, int nset);
 template <typename T> int launch_row_streams(const OpArgs<T> &a, hipStream_t s, int64_t *nblocks);
 template <typename T> int launch_col_inv_streams(const OpArgs<T> &a, hipStream_t s);
 // mix[b][6][N] of the nset sets from the half spectra spn[det][0..N/2]; mix32 may be null

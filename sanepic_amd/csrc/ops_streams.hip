@@ -96,118 +96,187 @@ __global__ __launch_bounds__(256) void k_col_fwd_st(OpArgs<T> a) {
   for (int s = 0; s < 16; s++) out[(int64_t)(t + TS * s) * N1 + n1] = cmul(v[s], tw_next<V>(tr));
 }
 
-// Row pass of the sets: 3 x 256 threads hold the same row of a set's three
-// streams; after the forward FFTs the spectra X_k pass through the LDS (in
-// halves of 8 values a thread in FP64, whose 3 x 34 KB hold no more) and
-// thread group k forms U_k = sum_j H_kj X_j in place of the product with W.
-// Three streams in one block, since a pass of its own for the mixing would
-// read and write them once more (16 of then 32 bytes a sample and stream).
-// Blocks take the same row of all of a set's pairs back to back, so the six
-// rows of H come from L2 for all but the first.
-template <typename T, int LOG2N1>
-__global__ __launch_bounds__(768) void k_row_mix(OpArgs<T> a) {
+// Threads of a stream in the row pass: 16 values each of a row, one wave at
+// least.  A CU's vector and LDS pipes serve the three streams of a block in
+// turn, so a block holds no more rows than it must: at 4 detectors x 1 segment
+// of 2^13 samples eight rows of 512 in 3 x 256 threads took 39 us on two CUs,
+// two rows in 3 x 64 threads take 10.7 us on eight (a row pass of the four
+// detectors 15 us).
+template <int LOG2N1>
+constexpr int row_group() {
+  return LOG2N1 <= 10 ? 64 : 1 << (LOG2N1 - 4);
+}
+
+// What thread group k of row block lb works on: first the sets' blocks, whose
+// groups hold the same rows of a set's three streams, then the detectors on
+// their own (OWN), three rows' blocks of them in turn (live: false past the last).
+// Blocks take the same rows of all of a stream's pairs back to back, so the
+// rows of H or W come from L2 for all but the first.
+struct RowAt {
+  int64_t row;   // of the stream's buffer: stream, pair and N1-point row
+  int64_t k2;
+  int64_t j;     // pair
+  int64_t wrow;  // first entry of the weights' row (H_00 of a set)
+  int32_t set;   // set, or -1 and
+  int32_t det;   // the detector
+  bool live;
+};
+template <bool OWN, typename T>
+__device__ __forceinline__ RowAt row_at(const OpArgs<T> &a, int64_t lb, int k, int b, int B) {
+  const int64_t N1 = a.g.N1, N = a.g.N, ppd = a.g.ppd, per = ppd * (a.g.N2 / B), nmix = a.nset * per;
+  RowAt w;
+  const bool mixed = !OWN || lb < nmix;
+  const int64_t nown = (a.nvs - 3 * (int64_t)a.nset) * per;
+  int64_t o = mixed ? lb : 3 * (lb - nmix) + k;
+  w.live = mixed || o < nown;
+  if (!w.live) o = nown - 1;  // a group without rows of its own still joins the barriers
+  const int64_t u = o / per, r = o % per;
+  const int64_t v = mixed ? 3 * u + k : 3 * (int64_t)a.nset + u;
+  w.j = r % ppd;
+  w.k2 = r / ppd * B + b;
+  w.row = (v * ppd + w.j) * N + w.k2 * N1;
+  w.set = mixed ? (int32_t)u : -1;
+  w.det = mixed ? 0 : a.vs[v].det;
+  w.wrow = (mixed ? 6 * u : (int64_t)w.det) * N + w.k2 * N1;
+  return w;
+}
+
+// Row pass of the sets: after the forward FFTs the spectra X_k of a set pass through the
+// LDS (in halves of 8 values a thread in FP64, whose 3 x 34 KB hold no more at
+// 4096) and thread group k forms U_k = sum_j H_kj X_j in place of the product
+// with W.  Three streams in one block, since a pass of its own for the mixing
+// would read and write them once more (16 of then 32 bytes a sample and
+// stream).  OWN: the detectors on their own in the same launch (row_merged).
+template <typename T, int LOG2N1, bool OWN>
+__global__ __launch_bounds__(3 * row_group<LOG2N1>()) void k_row_mix(OpArgs<T> a) {
   using V = VT<T>;
-  constexpr int N1 = 1 << LOG2N1, TS = N1 / 16, B = 256 / TS;
+  constexpr int G = row_group<LOG2N1>(), N1 = 1 << LOG2N1, TS = N1 / 16, B = G / TS;
   constexpr int HB = sizeof(T) == 8 ? 8 : 16;  // values exchanged at a time
-  static_assert(LdsSize<LOG2N1, B>::value <= kLds, "LDS");
-  static_assert(HB * 256 * sizeof(V) <= kLds * sizeof(LdsE<V>), "exchange");
-  __shared__ LdsE<V> lds[3 * kLds];
-  const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = threadIdx.x & 255, b = tid % B, t = tid / B;
-  const int p = k == 2 ? 0 : k + 1, q = k == 0 ? 2 : k - 1;  // the other two streams
-  const int64_t N = a.g.N, ppd = a.g.ppd, nrb = a.g.N2 / B, per = ppd * nrb;
-  const int64_t lb = logical_block(a.xcd), set = lb / per, r = lb % per;
-  const int64_t rb = r / ppd, j = r % ppd, k2 = rb * B + b;
-  const int64_t base = ((3 * set + k) * ppd + j) * N + k2 * N1;
+  constexpr int R = LdsSize<LOG2N1, B>::value;  // a stream's region
+  static_assert(HB * G * sizeof(V) <= R * sizeof(LdsE<V>), "exchange");
+  __shared__ LdsE<V> lds[3 * R];
+  const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / G), tid = threadIdx.x % G, b = tid % B, t = tid / B;
+  const RowAt at = row_at<OWN>(a, logical_block(a.xcd), k, b, B);
+  V *row = OWN ? a.buf + at.row : a.buf;  // written out: one form or the other spills (10 registers at N1 = 4096)
+  const int64_t base = OWN ? 0 : at.row;
   V v[16];
 #pragma unroll
-  for (int i = 0; i < 16; i++) v[i] = a.buf[base + t + TS * i];
-  LdsE<V> *own = lds + k * kLds;
+  for (int i = 0; i < 16; i++) v[i] = row[base + t + TS * i];
+  LdsE<V> *own = lds + k * R;
   fft_reg<V, -1, LOG2N1, B>(v, t, own + b, a.tw4096);
-  // H_kk, H_kp, H_kq: entry (i, j), i <= j, is the (3 i - i (i - 1) / 2 + j - i)-th
-  auto hrow = [&](int x, int y) {
-    const int i = x < y ? x : y, l = x < y ? y : x;
-    return a.mix + (set * 6 + (3 * i - i * (i - 1) / 2 + l - i)) * N + k2 * N1;
-  };
-  const T *hk = hrow(k, k), *hp = hrow(k, p), *hq = hrow(k, q);
-  V *ek = reinterpret_cast<V *>(own);
-  const V *ep = reinterpret_cast<const V *>(lds + p * kLds), *eq = reinterpret_cast<const V *>(lds + q * kLds);
+  if (OWN && at.set < 0) {
+    const T *w = a.wt + at.wrow;
 #pragma unroll
-  for (int h = 0; h < 16 / HB; h++) {
-    __syncthreads();  // the FFT's (or the last half's) LDS reads are done
+    for (int s = 0; s < 16; s++) {
+      const T ws = w[t + TS * s];
+      v[s] = mk<V>(v[s].x * ws, v[s].y * ws);
+    }
+  } else {
+    // H_kk, H_kp, H_kq: entry (i, j), i <= j, is the (3 i - i (i - 1) / 2 + j - i)-th
+    const int p = k == 2 ? 0 : k + 1, q = k == 0 ? 2 : k - 1;  // the other two streams
+    auto hrow = [&](int x, int y) {
+      const int i = x < y ? x : y, l = x < y ? y : x;
+      const int64_t e = 3 * i - i * (i - 1) / 2 + l - i;
+      return OWN ? a.mix + at.wrow + e * a.g.N : a.mix + ((int64_t)at.set * 6 + e) * a.g.N + at.k2 * N1;
+    };
+    const T *hk = hrow(k, k), *hp = hrow(k, p), *hq = hrow(k, q);
+    V *ek = reinterpret_cast<V *>(own);
+    const V *ep = reinterpret_cast<const V *>(lds + p * R), *eq = reinterpret_cast<const V *>(lds + q * R);
 #pragma unroll
-    for (int s = 0; s < HB; s++) ek[s * 256 + tid] = v[h * HB + s];
-    __syncthreads();
+    for (int h = 0; h < 16 / HB; h++) {
+      __syncthreads();  // the FFT's (or the last half's) LDS reads are done
 #pragma unroll
-    for (int s = 0; s < HB; s++) {
-      const int k1 = t + TS * (h * HB + s);
-      const V x = v[h * HB + s], xp = ep[s * 256 + tid], xq = eq[s * 256 + tid];
-      const T wk = hk[k1], wp = hp[k1], wq = hq[k1];
-      v[h * HB + s] = mk<V>(fma(wq, xq.x, fma(wp, xp.x, wk * x.x)), fma(wq, xq.y, fma(wp, xp.y, wk * x.y)));
+      for (int s = 0; s < HB; s++) ek[s * G + tid] = v[h * HB + s];
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < HB; s++) {
+        const int k1 = t + TS * (h * HB + s);
+        const V x = v[h * HB + s], xp = ep[s * G + tid], xq = eq[s * G + tid];
+        const T wk = hk[k1], wp = hp[k1], wq = hq[k1];
+        v[h * HB + s] = mk<V>(fma(wq, xq.x, fma(wp, xp.x, wk * x.x)), fma(wq, xq.y, fma(wp, xp.y, wk * x.y)));
+      }
     }
   }
   fft_reg<V, +1, LOG2N1, B>(v, t, own + b, a.tw4096);
-  TwRun tr = tw_run<+1>(a.twlo64, a.twhi64, (int64_t)t * k2, (int64_t)TS * k2);
+  if (OWN && !at.live) return;
+  TwRun tr = tw_run<+1>(a.twlo64, a.twhi64, (int64_t)t * at.k2, (int64_t)TS * at.k2);
 #pragma unroll
-  for (int s = 0; s < 16; s++) a.buf[base + t + TS * s] = cmul(v[s], tw_next<V>(tr));
+  for (int s = 0; s < 16; s++) row[base + t + TS * s] = cmul(v[s], tw_next<V>(tr));
 }
 
-// chi2 of the sets against each detector's own data spectrum: the forward
-// half of k_row_mix (rows read, not written), then the residuals
-// D_d - (X_0 + c_d X_1 + s_d X_2) of the detectors k, k + 3, ... in thread
-// group k.  A launch of its own before k_row_mix: with both in one kernel
-// the spectra, the data and the mixed values together spilled 98-225
-// registers a lane (1533 us; now 515 + 286 us at 16 detectors x 2^24 samples).
-template <int LOG2N1>
-__global__ __launch_bounds__(768) void k_row_chi(OpArgs<double> a) {
+// chi2 against each detector's own data spectrum: the forward half of
+// k_row_mix (rows read, not written), then the residuals
+// D_d - (X_0 + c_d X_1 + s_d X_2) of a set's detectors k, k + 3, ... in thread
+// group k, D_d - X of a detector on its own.  A launch of its own before
+// k_row_mix: with both in one kernel the spectra, the data and the mixed
+// values together spilled 98-225 registers a lane (1533 us; now 515 + 286 us at
+// 16 detectors x 2^24 samples).
+template <int LOG2N1, bool OWN>
+__global__ __launch_bounds__(3 * row_group<LOG2N1>()) void k_row_chi(OpArgs<double> a) {
   using V = double2;
-  constexpr int N1 = 1 << LOG2N1, TS = N1 / 16, B = 256 / TS, HB = 8;
-  static_assert(LdsSize<LOG2N1, B>::value <= kLds && HB * 256 * sizeof(V) <= kLds * sizeof(double), "LDS");
-  __shared__ double lds[3 * kLds];
-  __shared__ double red[12];
-  const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = threadIdx.x & 255, b = tid % B, t = tid / B;
-  const int64_t N = a.g.N, ppd = a.g.ppd, nrb = a.g.N2 / B, per = ppd * nrb;
-  const int64_t lb = logical_block(a.xcd), set = lb / per, r = lb % per;
-  const int64_t rb = r / ppd, j = r % ppd, k2 = rb * B + b;
-  const V *row = a.buf + ((3 * set + k) * ppd + j) * N + k2 * N1;
+  constexpr int G = row_group<LOG2N1>(), N1 = 1 << LOG2N1, TS = N1 / 16, B = G / TS, HB = 8;
+  constexpr int R = LdsSize<LOG2N1, B>::value, NW = 3 * G / 64;
+  static_assert(HB * G * sizeof(V) <= R * sizeof(double), "LDS");
+  __shared__ double lds[3 * R];
+  __shared__ double red[NW];
+  const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / G), tid = threadIdx.x % G, b = tid % B, t = tid / B;
+  const int64_t N = a.g.N, ppd = a.g.ppd, lb = logical_block(a.xcd);
+  const RowAt at = row_at<OWN>(a, lb, k, b, B);
+  const V *row = a.buf + at.row;
   V v[16];
 #pragma unroll
   for (int i = 0; i < 16; i++) v[i] = row[t + TS * i];
-  fft_reg<V, -1, LOG2N1, B>(v, t, lds + k * kLds + b, a.tw4096);
-  V *own = reinterpret_cast<V *>(lds + k * kLds);
-  const V *e0 = reinterpret_cast<const V *>(lds), *e1 = reinterpret_cast<const V *>(lds + kLds),
-          *e2 = reinterpret_cast<const V *>(lds + 2 * kLds);
-  const int d0 = a.sbeg[set] + k, d1 = a.sbeg[set + 1];
+  fft_reg<V, -1, LOG2N1, B>(v, t, lds + k * R + b, a.tw4096);
+  const bool dc = at.k2 == 0;  // bins 0 and N/2 are counted twice by the reference's per-segment sum
   double chi = 0.0;
+  if (OWN && at.set < 0) {
+    const V *D = a.dspec + ((int64_t)at.det * ppd + at.j) * N + at.k2 * N1;
+    const double *w = a.wt + at.wrow;
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
-    __syncthreads();
+    for (int s = 0; s < 16; s++) {
+      const int k1 = t + TS * s;
+      const V d = D[k1];
+      const double rx = d.x - v[s].x, ry = d.y - v[s].y;
+      double c = w[k1] * (rx * rx + ry * ry);
+      if (dc && (k1 == 0 || k1 == N1 / 2)) c += c;
+      chi += c;
+    }
+    if (!at.live) chi = 0.0;
+  } else {
+    V *own = reinterpret_cast<V *>(lds + k * R);
+    const V *e0 = reinterpret_cast<const V *>(lds), *e1 = reinterpret_cast<const V *>(lds + R),
+            *e2 = reinterpret_cast<const V *>(lds + 2 * R);
+    const int d0 = a.sbeg[at.set] + k, d1 = a.sbeg[at.set + 1];
 #pragma unroll
-    for (int s = 0; s < HB; s++) own[s * 256 + tid] = v[h * HB + s];
-    __syncthreads();
+    for (int h = 0; h < 2; h++) {
+      __syncthreads();
 #pragma unroll
-    for (int g = 0; g < HB; g += 4) {  // four bins: their spectra stay in registers over the detectors
+      for (int s = 0; s < HB; s++) own[s * G + tid] = v[h * HB + s];
+      __syncthreads();
+#pragma unroll
+      for (int g = 0; g < HB; g += 4) {  // four bins: their spectra stay in registers over the detectors
 #pragma unroll 1
-      for (int d = d0; d < d1; d += 3) {
-        const SkyDet sd = a.sdet[d];
-        const int64_t at = k2 * N1 + t + TS * (h * HB + g);
-        const V *D = a.dspec + ((int64_t)sd.det * ppd + j) * N + at;
-        const double *w = a.wt + (int64_t)sd.det * N + at;
-        V dv[4];
-        double wv[4];
+        for (int d = d0; d < d1; d += 3) {
+          const SkyDet sd = a.sdet[d];
+          const int64_t o = at.k2 * N1 + t + TS * (h * HB + g);
+          const V *D = a.dspec + ((int64_t)sd.det * ppd + at.j) * N + o;
+          const double *w = a.wt + (int64_t)sd.det * N + o;
+          V dv[4];
+          double wv[4];
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-          dv[s] = D[TS * s];
-          wv[s] = w[TS * s];
-        }
+          for (int s = 0; s < 4; s++) {
+            dv[s] = D[TS * s];
+            wv[s] = w[TS * s];
+          }
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-          const int e = (g + s) * 256 + tid, k1 = t + TS * (h * HB + g + s);
-          const double rx = dv[s].x - (e0[e].x + (sd.c * e1[e].x + sd.s * e2[e].x));
-          const double ry = dv[s].y - (e0[e].y + (sd.c * e1[e].y + sd.s * e2[e].y));
-          double c = wv[s] * (rx * rx + ry * ry);
-          // bins 0 and N/2 are counted twice by the reference's per-segment sum
-          if (k2 == 0 && (k1 == 0 || k1 == N1 / 2)) c += c;
-          chi += c;
+          for (int s = 0; s < 4; s++) {
+            const int e = (g + s) * G + tid, k1 = t + TS * (h * HB + g + s);
+            const double rx = dv[s].x - (e0[e].x + (sd.c * e1[e].x + sd.s * e2[e].x));
+            const double ry = dv[s].y - (e0[e].y + (sd.c * e1[e].y + sd.s * e2[e].y));
+            double c = wv[s] * (rx * rx + ry * ry);
+            if (dc && (k1 == 0 || k1 == N1 / 2)) c += c;
+            chi += c;
+          }
         }
       }
     }
@@ -218,8 +287,8 @@ __global__ __launch_bounds__(768) void k_row_chi(OpArgs<double> a) {
   __syncthreads();
   if (threadIdx.x == 0) {
     double tot = 0.0;
-    for (int i = 0; i < 12; i++) tot += red[i];
-    a.chi2part[a.chi2off + lb] = tot;
+    for (int i = 0; i < NW; i++) tot += red[i];
+    a.chi2part[lb] = tot;
   }
 }
 
@@ -390,30 +459,52 @@ int launch_col_fwd_streams(const OpArgs<T> &a, hipStream_t s) {
 #undef CS
 }
 
+// Whether the detectors on their own share the sets' row launch.  In small
+// contexts a launch after it costs more than their rows (4 + 1 detectors x 4
+// segments of 2^13 samples: 87 us an iteration with two launches, 72 with one,
+// 79 with one stream per detector); in large ones the rows of one wave or two a
+// stream lose to blocks of 256 threads (8 + 9 x 8 x 2^18: 894 us, 958 with one
+// launch), and at N1 = 4096 the common kernel would spill 65 registers.
+static bool row_merged(const PairGeom &g, int nvs, int nset) {
+  return nvs > 3 * nset && g.log2N1 <= 11 && nvs * g.ppd * g.N < kStreamsSmall;
+}
+
+int64_t stream_row_blocks(const PairGeom &g, int nvs, int nset) {
+  const int64_t rows = g.ppd * (g.N / 4096), n = rows * (g.log2N1 <= 10 ? 4 : g.log2N1 == 11 ? 2 : 1);
+  const int64_t own = nvs - 3 * (int64_t)nset;
+  return nset * n + (row_merged(g, nvs, nset) ? (own * n + 2) / 3 : own * rows);
+}
+
 template <typename T>
 int launch_row_streams(const OpArgs<T> &a, hipStream_t s, int64_t *nblocks) {
-  const int64_t rows = a.g.ppd * (a.g.N / 4096), nmix = a.nset * rows, nown = (a.nvs - 3 * (int64_t)a.nset) * rows;
-  const bool chi = (a.mode & ROW_CHI2) != 0;
-  if (nblocks) *nblocks = nmix + nown;
-  if (nmix > 0x7fffffffLL) return -1;
+  const bool chi = (a.mode & ROW_CHI2) != 0, merged = row_merged(a.g, a.nvs, a.nset);
+  const int64_t nb = stream_row_blocks(a.g, a.nvs, a.nset);
+  const int64_t nown = merged ? 0 : (a.nvs - 3 * (int64_t)a.nset) * a.g.ppd * (a.g.N / 4096), nmix = nb - nown;
+  if (nblocks) *nblocks = nb;
   if (chi && sizeof(T) != 8) return -2;
-#define RM(L)                                                                                             \
-  case L:                                                                                                 \
-    if constexpr (sizeof(T) == 8)                                                                         \
-      if (chi) hipLaunchKernelGGL(k_row_chi<L>, dim3((unsigned)nmix), dim3(768), 0, s, a);                \
-    hipLaunchKernelGGL((k_row_mix<T, L>), dim3((unsigned)nmix), dim3(768), 0, s, a);                      \
+#define RM1(L, OWN)                                                                     \
+  do {                                                                                  \
+    if constexpr (sizeof(T) == 8)                                                       \
+      if (chi && launch1(k_row_chi<L, OWN>, nmix, s, a, 3 * row_group<L>())) return -1; \
+    if (launch1(k_row_mix<T, L, OWN>, nmix, s, a, 3 * row_group<L>())) return -1;       \
+  } while (0)
+#define RM(L)                  \
+  case L:                      \
+    if (merged) RM1(L, true);  \
+    else RM1(L, false);        \
     break;
   switch (a.g.log2N1) {
-    RM(9) RM(10) RM(11) RM(12)
+    RM(9) RM(10) RM(11)
+    case 12: RM1(12, false); break;
     default: return -2;
   }
 #undef RM
-  if (hipGetLastError() != hipSuccess) return -1;
+#undef RM1
   if (nown <= 0) return 0;
   OpArgs<T> o = a;
   o.g.npairs = nown / (a.g.N / 4096);
   o.g.pair0 = 0;
-  o.chi2off = a.chi2off + nmix;
+  o.chi2off = nmix;
   switch (a.g.log2N1) {
     case 9: return launch1(k_row_own<T, 9>, nown, s, o);
     case 10: return launch1(k_row_own<T, 10>, nown, s, o);
