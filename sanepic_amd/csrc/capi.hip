@@ -585,10 +585,6 @@ int sorted_turns(sanepic_ctx *c) {
   return 0;
 }
 
-}  // namespace sctx
-
-namespace {
-
 // Four-step split N1 = 2^log2n1 (the weight tables follow the split).
 int set_split(sanepic_ctx *c, int log2n1) {
   PairGeom &g = c->g;
@@ -617,6 +613,27 @@ int set_split(sanepic_ctx *c, int log2n1) {
   dfree(c, c->mix32, 6 * (int64_t)c->nset * c->ns);
   return c->pixelized ? sorted_turns(c) : 0;  // a split without run records
 }
+
+// The split of a context that is asked for none: rows of up to 4096, the
+// fewest columns passes can have.  Contexts that filter sets of streams take
+// rows of 1024 where the columns then fit a record pass (256 points): a row's
+// three streams are 192 threads instead of 768 that share a CU's pipes (4
+// detectors x 1 x 2^16 samples: 78 us an iteration with 4096, 66 with 1024; 16 x
+// 64 x 2^18: 943 and 936).  With detectors on their own only below the size
+// where these share the row launch: 8 + 9 x 8 x 2^18 take 868 us with 4096, 956
+// with 1024; 5 + 3 x 8 x 2^17 213 and 197.
+int default_split(const sanepic_ctx *c) {
+  const int l = c->g.log2N;
+  if (c->g.M != 1) return std::min(12, l - 4);
+  const int n1 = l - std::max(4, l - 12);
+  if (!c->nstream || l > 18) return n1;
+  if (c->nstream > 3 * c->nset && c->nstream * c->g.ppd * c->g.N >= kStreamsSmall) return n1;
+  return std::min(n1, 10);
+}
+
+}  // namespace sctx
+
+namespace {
 
 double pixel_eps() {
   const char *e = getenv("SANEPIC_PIXEL_EPS");
@@ -745,7 +762,7 @@ int create_context(const sanepic_config *cfg, sanepic_ctx **out, bool pointing) 
     g.log2N1 = l;
     g.log2N2 = 0;
   } else {
-    g.log2N1 = radix == 1 ? l - std::max(4, l - 12) : std::min(12, l - 4);
+    g.log2N1 = default_split(c);
     g.log2N2 = l - g.log2N1;
     g.N1 = int64_t(1) << g.log2N1;
     g.N2 = (int64_t)radix << g.log2N2;
@@ -1206,6 +1223,7 @@ int sanepic_pixelize(sanepic_ctx *c, int64_t *npix_out, int64_t *n_deferred) {
   trace_mark("pixelize: sorted angles");
   ACHK(c, build_items(c, ntot, c->items_nested && c->d_slot2pix != nullptr));
   ACHK(c, find_streams(c));
+  if (c->nstream) ACHK(c, set_split(c, default_split(c)));
   ACHK(c, build_runs(c));
   ACHK(c, sorted_turns(c));
   // a group keeps it for fetch_host_order, shared lines of sight until the set-up (drop_streams)
@@ -1249,7 +1267,9 @@ int sanepic_get_indpix(sanepic_ctx *c, int64_t *indpix) {
 int sanepic_set_fft_split(sanepic_ctx *c, int32_t log2_n1) {
   ACHK(c, check_ready(c, false));
   if (c->setup_done) return fail(c, SANEPIC_EINVAL, "the split is fixed by sanepic_setup");
-  return set_split(c, log2_n1);
+  ACHK(c, set_split(c, log2_n1));
+  c->split_chosen = true;
+  return SANEPIC_OK;
 }
 
 int sanepic_autotune(sanepic_ctx *c, const char *cache, int32_t *log2_n1, double *op_ms) {
@@ -1273,6 +1293,7 @@ int sanepic_autotune(sanepic_ctx *c, const char *cache, int32_t *log2_n1, double
     if (op_ms) *op_ms = 0.0;
     return SANEPIC_OK;
   }
+  c->split_chosen = true;
   hipDeviceProp_t prop{};
   HIPCHK(c, hipGetDeviceProperties(&prop, c->cfg.device));
   char key[512];

@@ -143,7 +143,8 @@ int drop_streams(sanepic_ctx *c) {
   c->ritems = ItemSet();
   c->nstream = c->nset = c->nline = 0;
   c->nrec = 0;
-  return build_runs(c);
+  ACHK(c, build_runs(c));
+  return c->split_chosen ? 0 : set_split(c, default_split(c));
 }
 
 template <typename T>

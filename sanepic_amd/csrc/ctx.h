@@ -251,6 +251,7 @@ struct sanepic_ctx {
   double *apply_x = nullptr, *apply_y = nullptr;  // [npix][nc] sanepic_apply's and sanepic_chi2's maps
   bool deflate = false;
   double *az = nullptr;
+  bool split_chosen = false;         // by the caller or the autotuner
   bool begun = false, setup_done = false, pixelized = false;
   bool prof = false;
   std::vector<std::tuple<int, hipEvent_t, hipEvent_t>> evs;
@@ -557,6 +558,8 @@ bool use_runs(const sanepic_ctx *c);
 // run layout; whether an operator application filters streams; its three
 // passes (run records out).
 int find_streams(sanepic_ctx *c);
+int set_split(sanepic_ctx *c, int log2n1);
+int default_split(const sanepic_ctx *c);
 int drop_streams(sanepic_ctx *c);
 bool use_streams(const sanepic_ctx *c);
 template <typename T> int run_streams(sanepic_ctx *c, OpArgs<T> a, bool chi2, int64_t *nb);

@@ -36,3 +36,40 @@ def test_rows_against_the_oracle(offsets, nseg, ns, split, streams):
         print(f"  precision {prec}: A x {e:.1e}, chi2 {e_c:.1e}", flush=True)
         assert e < tol and e_c < 1e-10
         ctx.close()
+
+
+def _bits(cfg, ds, split, x, recal=False):
+    ctx = sanepic_amd.Context(cfg.nside, cfg.ndet, cfg.nseg, cfg.ns)
+    ctx.load(cfg, ds)
+    ctx.pixelize()
+    if split is not None:
+        ctx.set_fft_split(split)
+    if recal:
+        ctx.set_recalib(True)
+    ctx.setup()
+    y = ctx.apply(x)
+    ctx.close()
+    return y
+
+
+@pytest.mark.parametrize("offsets,nseg,ns,shared,plain", [
+    ([A] * 4, 2, 2 ** 13, 9, 9),
+    ([A] * 4, 2, 2 ** 16, 10, 12),
+    ([A] * 4, 1, 2 ** 18, 10, 12),
+    ([A] * 4, 1, 2 ** 19, 12, 12),
+    ([A] * 4 + [B], 3, 2 ** 16, 10, 12),
+    ([A] * 4 + [B], 17, 2 ** 17, 12, 12),
+])
+def test_split_of_shared_lines(offsets, nseg, ns, shared, plain):
+    """Rows of 1024 where the operator filters sets of streams, unless the
+    caller chose; the usual ones when a calibration takes the sharing away."""
+    print("split", len(offsets), nseg, ns, flush=True)
+    cfg, ds = _case(offsets, nseg, ns, nside=8)
+    ctx = _ctx(cfg, ds)
+    x = np.random.default_rng(8).standard_normal(3 * ctx.npix)
+    ctx.close()
+    assert np.array_equal(_bits(cfg, ds, None, x), _bits(cfg, ds, shared, x))
+    assert np.array_equal(_bits(cfg, ds, None, x, True), _bits(cfg, ds, plain, x, True))
+    if ns == 2 ** 16:
+        kept = _bits(cfg, ds, 11, x, True)
+        assert not np.array_equal(kept, _bits(cfg, ds, None, x, True))
