@@ -35,9 +35,16 @@ bool use_streams(const sanepic_ctx *c) {
 // the rounding of those sums (2e-12 in A x at 2^19 samples of a plate at
 // 0.048 rad a sample, growing with t; below 1e-14 for the bounded angles).
 // Sets of four or more detectors become three streams; every other detector
-// stays a stream of its own.  Used when that leaves at most four streams for
-// every five detectors: a detector on its own costs the same either way but
-// for its records' two idle sums (40 instead of 24 bytes a run).
+// stays a stream of its own, which costs it more than the usual passes: its
+// records hold two idle sums (40 instead of 24 bytes a run in FP64) and its
+// record pass batches its loads less, 1.3 to 1.4 times a detector's share of an
+// FP64 iteration (10 sharing + 25, 4 x 2^17: 725 us with one stream each, 791
+// shared; 16 + 48, 2 x 2^18: 1590 and 1645).  In FP64 a set pays where own
+// detectors times 3/2 and its three streams stay below the number of detectors
+// (16 + 25: 837 and 761; 8 + 9: 366 and 308).  Half the width of records and
+// angles halves that surcharge: a mixed context shares when that leaves at most
+// four streams for every five detectors (16 + 48: 1141 and 1082; 10 + 25: 526
+// and 530).
 int find_streams(sanepic_ctx *c) {
   if (!c->runs || c->pin_owner || !c->sub.empty() || c->single || c->zsorted || c->nc != 3 || c->g.M != 1 ||
       c->pregather || c->recal || c->chunk != 0 || !c->ang64 || c->ndet < 4 || c->ndet > 65535 || c->ns % 16 != 0 ||
@@ -94,7 +101,9 @@ int find_streams(sanepic_ctx *c) {
   const int32_t nset = line;
   for (int32_t d = 0; d < (int32_t)c->ndet; d++)
     if (!taken[(size_t)d]) vs.push_back(SkyStream{d, line++, 3, 0, 0});
-  if (nset == 0 || 5 * (int64_t)vs.size() > 4 * c->ndet) return 0;
+  const int64_t nvs = (int64_t)vs.size(), nown = nvs - 3 * nset;
+  if (nset == 0 || 5 * nvs > 4 * c->ndet) return 0;
+  if (c->cfg.precision == SANEPIC_FP64 && 6 * nset + 3 * nown >= 2 * c->ndet) return 0;
   c->nstream = (int)vs.size();
   c->nset = nset;
   c->nline = line;

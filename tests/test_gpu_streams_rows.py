@@ -73,3 +73,26 @@ def test_split_of_shared_lines(offsets, nseg, ns, shared, plain):
     if ns == 2 ** 16:
         kept = _bits(cfg, ds, 11, x, True)
         assert not np.array_equal(kept, _bits(cfg, ds, None, x, True))
+
+
+@pytest.mark.parametrize("nshare,nown,fp64,mixed", [
+    (4, 0, (3, 1), (3, 1)),
+    (4, 1, (4, 2), (4, 2)),
+    (5, 3, (6, 4), (6, 4)),
+    (6, 5, (8, 6), (8, 6)),
+    (6, 6, (12, 12), (9, 7)),
+    (7, 8, (15, 15), (11, 9)),
+    (7, 13, (20, 20), (16, 14)),
+    (4, 2, (6, 6), (6, 6)),
+])
+def test_sharing_pays(nshare, nown, fp64, mixed):
+    """A detector on its own costs more beside a set: an FP64 context with many
+    of them keeps one stream each."""
+    off = [A] * nshare + [(0.05 * (k + 1), 0.3 - 0.02 * k) for k in range(nown)]
+    cfg, ds = _case(off, 1, 2 ** 13, nside=8)
+    for prec, want in ((sanepic_amd.FP64, fp64), (sanepic_amd.MIXED, mixed)):
+        ctx = sanepic_amd.Context(cfg.nside, cfg.ndet, cfg.nseg, cfg.ns, precision=prec)
+        ctx.load(cfg, ds)
+        ctx.pixelize()
+        assert ctx.streams() == want
+        ctx.close()
