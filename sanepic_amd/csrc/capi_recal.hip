@@ -133,8 +133,10 @@ int sanepic_set_recalib(sanepic_ctx *c, int32_t on) {
   if (!c->sub.empty())
     return fail(c, SANEPIC_EINVAL, "relative calibration needs one segment length for every detector");
   if (c->setup_done) return fail(c, SANEPIC_EINVAL, "sanepic_set_recalib belongs before sanepic_setup");
-  c->recal = on != 0;
-  if (!c->recal) return SANEPIC_OK;
+  if (!on) {
+    c->recal = false;
+    return SANEPIC_OK;
+  }
   const int64_t nblk = c->ndet * c->nseg;
   c->h_gain.assign(nblk, 1.0);
   c->h_gain32.assign(nblk, 1.0f);
@@ -146,6 +148,7 @@ int sanepic_set_recalib(sanepic_ctx *c, int32_t on) {
     ACHK(c, drop_streams(c));
     ACHK(c, sorted_turns(c));
   }
+  c->recal = true;  // only now: after a failure above the context is as it was, but for the streams
   return SANEPIC_OK;
 }
 

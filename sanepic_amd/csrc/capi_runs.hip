@@ -90,9 +90,11 @@ namespace sctx {
 
 bool use_runs(const sanepic_ctx *c) {
   // the inverse column pass writes records when its 16-lane rows hold whole
-  // pieces: power-of-two lengths with at most 256 rows (16 columns a block)
+  // pieces: power-of-two lengths with at most 256 rows (16 columns a block).
+  // The records of shared lines of sight (one set for all detectors of a line,
+  // five sums each) are for the passes over streams only.
   return c->nrec > 0 && c->nc == 3 && !c->single && c->sub.empty() && !c->zsorted && c->g.M == 1 &&
-         c->g.log2N2 <= 8;
+         c->g.log2N2 <= 8 && (c->nstream == 0 || (!c->pregather && !c->recal && c->chunk == 0));
 }
 
 int build_runs(sanepic_ctx *c) {

@@ -23,7 +23,8 @@ namespace sctx {
 
 bool use_streams(const sanepic_ctx *c) {
   // the gather runs in the column pass, without gains; whole launches only
-  return c->nstream > 0 && use_runs(c) && !c->pregather && !c->recal && c->chunk == 0;
+  // (use_runs is false otherwise)
+  return c->nstream > 0 && use_runs(c);
 }
 
 // Finds the sets (equal offsets, and the same pixels sample by sample: a
