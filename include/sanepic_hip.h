@@ -314,7 +314,8 @@ int sanepic_true_residual(sanepic_ctx *ctx, double *rel);
 int sanepic_set_profiling(sanepic_ctx *ctx, int32_t on);
 int sanepic_kernel_time(sanepic_ctx *ctx, int32_t which, double *ms,
                         int64_t *count);
-/* Device bytes held by the context. */
+/* Device bytes held by the context: its buffers, and slabs they were cut from
+ * that hold none at the moment (the unused parts of slabs in use not counted). */
 int sanepic_device_bytes(sanepic_ctx *ctx, int64_t *bytes);
 /* The run layout of P^T (no counterpart in the reference, whose do_PtNd
  * scatters sample by sample, sanepic.cc:2584-2611): *nrec = runs of

@@ -1676,6 +1676,7 @@ int sanepic_setup(sanepic_ctx *c) {
   trace_mark("setup: TOD uploads done");
   ACHK(c, setup_data(c));
   if (!keep_temporaries(c)) flush_frees(c);
+  c->arena.trim();
   trace_mark("setup: deferred frees");
   c->setup_done = true;
   return SANEPIC_OK;
@@ -1994,7 +1995,7 @@ int sanepic_device_bytes(sanepic_ctx *c, int64_t *bytes) {
   if (!c) return SANEPIC_EINVAL;
   int64_t b = c->bytes;
   for (sanepic_ctx *s : c->sub) b += s->bytes;
-  *bytes = b;
+  *bytes = b + c->arena.idle();
   return SANEPIC_OK;
 }
 

@@ -359,6 +359,7 @@ int group_setup(sanepic_ctx *c) {
     flush_frees(s);
     s->setup_done = true;
   }
+  c->arena.trim();  // the groups' TOD and temporaries
   const int64_t npix = c->npix;
   ACHK(c, dalloc(c, c->b_raw, 3 * npix));
   ACHK(c, dalloc(c, c->b, 3 * npix));
@@ -402,6 +403,7 @@ int group_setup(sanepic_ctx *c) {
   HIPCHK(c, hipStreamSynchronize(c->st));
   trace_mark("group setup: union sums");
   flush_frees(c);
+  c->arena.trim();
   trace_mark("group setup: deferred frees");
   c->setup_done = true;
   return SANEPIC_OK;

@@ -38,20 +38,26 @@ struct ItemSet {
 // size (below 1 MB the runtime has its own slabs: 1 us each): a run of 4
 // detectors x 6 x 2^17 samples from host buffers to maps spent 7 of its 13 ms
 // on a hundred of them (8.1 ms with the slabs).  Blocks given back serve later requests of
-// the same context (best fit, neighbours merged); the slabs are freed with it.
-// One host thread per context, as everything here; blocks are given back only
-// once the work that reads them is done.
+// the same context (best fit, neighbours merged).  Slabs without a block in use
+// go back to the device when a set-up ends and when an allocation fails, the
+// others with the context.  One host thread per context, as everything here;
+// blocks are given back only once the work that reads them is done.
 struct Arena {
   std::map<char *, int64_t> slabs, spare;        // address -> bytes
   std::unordered_map<void *, int64_t> used;
   static constexpr int64_t kAlign = 4096;
+  static constexpr int64_t kSlab = int64_t(1) << 28;  // larger slabs were made for one request
 
-  // from the spare blocks; null if none fits
+  // from the spare blocks; null if none fits.  A block beyond the size of a
+  // common slab serves only requests of half its size: a small buffer in it
+  // would keep gigabytes (a detector group's TOD) from the device.
   void *take(int64_t bytes) {
     const int64_t n = (bytes + kAlign - 1) / kAlign * kAlign;
     auto best = spare.end();
     for (auto it = spare.begin(); it != spare.end(); ++it)
-      if (it->second >= n && (best == spare.end() || it->second < best->second)) best = it;
+      if (it->second >= n && (it->second <= kSlab || it->second <= 2 * n) &&
+          (best == spare.end() || it->second < best->second))
+        best = it;
     if (best == spare.end()) return nullptr;
     char *p = best->first;
     const int64_t rest = best->second - n;
@@ -97,6 +103,28 @@ struct Arena {
     }
     spare[p] = n;
     return true;
+  }
+  // bytes of the slabs without a block in use
+  int64_t idle() const {
+    int64_t n = 0;
+    for (auto &b : spare) {
+      auto s = slabs.find(b.first);
+      if (s != slabs.end() && s->second == b.second) n += b.second;
+    }
+    return n;
+  }
+  // gives those back to the device
+  void trim() {
+    for (auto b = spare.begin(); b != spare.end();) {
+      auto s = slabs.find(b->first);
+      if (s != slabs.end() && s->second == b->second) {
+        (void)hipFree(b->first);
+        slabs.erase(s);
+        b = spare.erase(b);
+      } else {
+        ++b;
+      }
+    }
   }
   void free_all() {
     for (auto &s : slabs) (void)hipFree(s.first);
@@ -347,16 +375,18 @@ inline Arena &arena_of(sanepic_ctx *c) { return c->pin_owner ? c->pin_owner->are
 // size: the groups' temporaries, released one group after the other, serve the
 // next group, and a release of even the smallest to the runtime would wait for
 // the TOD uploads in flight (64 detectors x 2^24 samples: 0.12 s in the first
-// group's pixelisation).
+// group's pixelisation).  Larger ones take a spare block if one fits, such as
+// the groups' temporaries during the parent's pixelisation, else the device.
 constexpr int64_t kArenaMin = int64_t(1) << 20, kArenaMax = int64_t(1) << 27;
 
 inline hipError_t dev_alloc(sanepic_ctx *c, void **v, int64_t bytes) {
-  if (!c->pin_owner && (bytes < kArenaMin || bytes >= kArenaMax)) return hipMalloc(v, (size_t)bytes);
+  if (!c->pin_owner && bytes < kArenaMin) return hipMalloc(v, (size_t)bytes);
   Arena &a = arena_of(c);
   *v = a.take(bytes);
   if (*v) return hipSuccess;
+  if (!c->pin_owner && bytes >= kArenaMax) return hipMalloc(v, (size_t)bytes);
   // a slab for a third of the context's per-sample state, 16 to 256 MB
-  const int64_t want = std::min<int64_t>(int64_t(1) << 28, std::max<int64_t>(int64_t(1) << 24, c->ntot * 32));
+  const int64_t want = std::min<int64_t>(Arena::kSlab, std::max<int64_t>(int64_t(1) << 24, c->ntot * 32));
   const hipError_t e = a.grow(bytes, want);
   if (e == hipSuccess) *v = a.take(bytes);
   return e;
@@ -374,11 +404,15 @@ inline int dalloc(sanepic_ctx *c, T *&p, int64_t n) {
   const int64_t bytes = (int64_t)((size_t)n * sizeof(T));
   void *v = nullptr;
   hipError_t e = dev_alloc(c, &v, bytes);
-  if (e != hipSuccess && !c->later.empty() && !c->pin_owner) {
-    // set-up temporaries kept past the set-up (keep_temporaries) go first
+  if (e != hipSuccess) {
+    // set-up temporaries kept past the set-up (keep_temporaries) and slabs
+    // without a block in use go first
     (void)hipGetLastError();
-    if (hipStreamSynchronize(c->st) != hipSuccess) (void)hipGetLastError();
-    flush_frees(c);
+    if (!c->later.empty() && !c->pin_owner) {
+      if (hipStreamSynchronize(c->st) != hipSuccess) (void)hipGetLastError();
+      flush_frees(c);
+    }
+    arena_of(c).trim();
     e = dev_alloc(c, &v, bytes);
   }
   if (e != hipSuccess) {
