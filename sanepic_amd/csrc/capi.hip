@@ -635,6 +635,10 @@ int default_split(const sanepic_ctx *c) {
 
 namespace {
 
+// Of the cached splits: raised when the passes change, so that timings of the
+// earlier kernels are not used.
+constexpr int kTuneKernels = 2;
+
 double pixel_eps() {
   const char *e = getenv("SANEPIC_PIXEL_EPS");
   if (e && *e) return atof(e);
@@ -1297,8 +1301,14 @@ int sanepic_autotune(sanepic_ctx *c, const char *cache, int32_t *log2_n1, double
   hipDeviceProp_t prop{};
   HIPCHK(c, hipGetDeviceProperties(&prop, c->cfg.device));
   char key[512];
-  snprintf(key, sizeof(key), "%s ns=%ld ndet=%ld nseg=%ld npix=%ld precision=%d", prop.gcnArchName, (long)c->ns,
-           (long)c->ndet, (long)c->nseg, (long)c->npix, (int)c->cfg.precision);
+  // everything that decides which passes an application runs: contexts of equal
+  // sizes filter sets of streams or detectors, write records or samples
+  snprintf(key, sizeof(key),
+           "%s kernels=%d ns=%ld ndet=%ld nseg=%ld npix=%ld precision=%d nc=%d sets=%d streams=%d runs=%d group=%d "
+           "gains=%d pregather=%d chunk=%ld zsort=%d",
+           prop.gcnArchName, kTuneKernels, (long)c->ns, (long)c->ndet, (long)c->nseg, (long)c->npix,
+           (int)c->cfg.precision, c->nc, c->nset, c->nstream, c->nrec > 0 ? 1 : 0, c->pin_owner ? 1 : 0,
+           c->recal ? 1 : 0, c->pregather ? 1 : 0, (long)c->chunk, c->zsorted ? 1 : 0);
   if (cache) {
     if (FILE *f = fopen(cache, "r")) {
       char line[640];
