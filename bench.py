@@ -63,6 +63,14 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
+def streams_option(shared):
+    """Whether contexts created from here on filter shared lines of sight."""
+    if shared:
+        os.environ.pop("SANEPIC_STREAMS", None)
+    else:
+        os.environ["SANEPIC_STREAMS"] = "0"
+
+
 def class_bytes_per_sample(precision, rps=0.0, ang64=16, sorted64=16, lines=1.0):
     """Algorithmic HBM bytes per TOD sample of each operator kernel class
     (reads + writes of its streams; the map gathers hit the caches).
@@ -339,6 +347,55 @@ def run_solve(cfg, pin, precision, precond, deflate, weights, steps, warmup, max
     return out
 
 
+def operator_figures(r, cfg, ntot, workload, label):
+    """Per-iteration and operator figures of an FP64 solve: samples per second,
+    the operator's time and algorithmic bytes, and the roofline of its dominant
+    kernel class (label: the operator's name in profiles/)."""
+    uneven = hasattr(cfg, "seglen")
+    kt = r["kernel_times"]
+    per = [(kt[k][0], kt[k][1], k) for k in range(4) if kt[k][1] > 0]
+    tot_ms, cnt_launch, dom = max(per)
+    # per operator application: with per-detector lengths one application
+    # launches each kernel class once per detector group
+    n_ops = max(kt[4][1], 1)
+    avg_ms = tot_ms / n_ops
+    nrec, runs_on = r["run_records"]
+    nstr, nline = r["streams"]
+    shared = nstr < cfg.ndet
+    nfilt = ntot * nstr // cfg.ndet  # samples of the filtered streams
+    rps = nrec / nfilt if runs_on else 0.0
+    names = CLASS_NAMES_RUNS if runs_on else CLASS_NAMES
+    cbs = class_bytes_per_sample("fp64", rps, r["fp64_angle_bytes"], r["fp64_sorted_angle_bytes"] or 16,
+                                 nline / nstr if shared else 1.0)
+    alg = nfilt * cbs[dom]  # algorithmic bytes of the dominant kernel class per operator application
+    achieved = alg / (avg_ms * 1e-3)
+    for k in range(4):
+        if kt[k][1]:
+            log(f"  {label} {names[k]}: {kt[k][0] / n_ops:.3f} ms per operator ({kt[k][1]} launches, "
+                f"{nfilt * cbs[k] / (kt[k][0] / n_ops * 1e-3) / 1e12:.2f} TB/s of algorithmic bytes)")
+    apply_ms = kt[4][0] / n_ops
+    lens = cfg.seglen if uneven else [cfg.ns] * cfg.ndet
+    # whole-operator algorithmic bytes: each filtered line's stream read once
+    # (int32 pixel + cos 2psi + sin 2psi), the per-detector noise weights, ~12
+    # map-vector passes of the CG in FP64
+    lines = ntot if not shared else ntot // cfg.ndet * nline
+    b_alg = lines * (4 + 2 * 8) + sum(L // 2 + 1 for L in lens) * 8 + 12 * 3 * r["npix"] * 8
+    traffic, traffic_src = read_traffic(workload, label, names[dom])
+    return {
+        "value": ntot / (r["ms_per_step"] * 1e-3),
+        "ms_per_step": r["ms_per_step"],
+        "operator_ms": apply_ms,
+        "operator_alg_bytes": b_alg,
+        "operator_frac_hbm": b_alg / (apply_ms * 1e-3) / HBM_PEAK,
+        "run_records": {"records": nrec, "per_sample": rps, "used": runs_on},
+        "streams": {"filtered": nstr, "lines_of_sight": nline, "detectors": cfg.ndet},
+        "roofline": {"bound": "hbm", "kernel": names[dom], "achieved": achieved / 1e9,
+                     "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": achieved / HBM_PEAK,
+                     "traffic": traffic, "traffic_source": traffic_src, "bytes_per_launch": alg,
+                     "ms_per_launch": avg_ms, "launches_per_operator": cnt_launch // n_ops},
+    }
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -409,7 +466,8 @@ def main():
     deflate = not args.no_deflate
     rf = args.mixed_refresh
 
-    # the headline: FP64 block-Jacobi, the reference's arithmetic
+    # the headline: FP64 block-Jacobi, the reference's arithmetic and one filtered stream per detector
+    streams_option(shared=False)
     head = run_solve(cfg, pin, "fp64", "block", False, None, args.steps, args.warmup, args.maxiter,
                      profile=True, reference=True, track_self=not args.no_map_track)
     ref_map, cnt = head["ref_map"], head["cnt"]
@@ -428,49 +486,32 @@ def main():
                                   args.maxiter, profile=False, net_nside=(record or {}).get("net_nside"),
                                   refresh=rf, fallback_growth=growth, keep_map=True,
                                   track=None if args.no_map_track else (ref_map, cnt))
+    # the library's own choice where detectors share a line of sight
+    streams_option(shared=True)
+    shared = {}
+    if not uneven:
+        time.sleep(args.settle)
+        r = run_solve(cfg, pin, "fp64", "block", False, None, args.steps, args.warmup, args.maxiter, profile=True,
+                      keep_map=True)
+        if r["streams"][0] < cfg.ndet:
+            shared["fp64"] = r
+            if "learned" in runs:
+                time.sleep(args.settle)
+                shared["learned"] = run_solve(cfg, pin, "mixed", "learned", deflate, weights, 2, 1, args.maxiter,
+                                              profile=False, net_nside=(record or {}).get("net_nside"), refresh=rf,
+                                              keep_map=True)
     pin.close()
 
-    kt = head["kernel_times"]
-    ms_per_step = head["ms_per_step"]
-    per = [(kt[k][0], kt[k][1], k) for k in range(4) if kt[k][1] > 0]
-    tot_ms, cnt_launch, dom = max(per)
-    # per operator application: with per-detector lengths one application
-    # launches each kernel class once per detector group
-    n_ops = max(kt[4][1], 1)
-    avg_ms = tot_ms / n_ops
-    nrec, runs_on = head["run_records"]
-    nstr, nline = head["streams"]
-    nfilt = ntot * nstr // cfg.ndet  # samples of the filtered streams
-    rps = nrec / nfilt if runs_on else 0.0
-    names = CLASS_NAMES_RUNS if runs_on else CLASS_NAMES
-    cbs = class_bytes_per_sample("fp64", rps, head["fp64_angle_bytes"],
-                                 head["fp64_sorted_angle_bytes"] or 16, nline / nstr if nstr < cfg.ndet else 1.0)
-    alg = nfilt * cbs[dom]  # algorithmic bytes of the dominant kernel class per operator application
-    achieved = alg / (avg_ms * 1e-3)
-    for k in range(4):
-        if kt[k][1]:
-            log(f"  {names[k]}: {kt[k][0] / n_ops:.3f} ms per operator ({kt[k][1]} launches, "
-                f"{nfilt * cbs[k] / (kt[k][0] / n_ops * 1e-3) / 1e12:.2f} TB/s of algorithmic bytes)")
-    apply_ms = kt[4][0] / max(kt[4][1], 1)
-    lens = cfg.seglen if uneven else [cfg.ns] * cfg.ndet
-    npix = head["npix"]
-
-    def b_alg(s):
-        # whole-operator algorithmic bytes: the stream of each line of sight
-        # read once (int32 pixel + cos 2psi + sin 2psi), the per-detector
-        # noise weights, ~12 map-vector passes of the CG in FP64
-        return ntot // cfg.ndet * nline * (4 + 2 * s) + sum(L // 2 + 1 for L in lens) * s + 12 * 3 * npix * 8
-
-    traffic, traffic_src = read_traffic(args.workload, "fp64", names[dom])
+    op = operator_figures(head, cfg, ntot, args.workload, "fp64")
     tts = head["time_to_solution_s"]
     out = {
         "metric": "time-to-1e-6 residual (s) + TOD samples/s per CG iter, NSIDE512 16det, 1 GPU",
-        "value": ntot / (ms_per_step * 1e-3),
+        "value": op["value"],
         "unit": "TOD samples/s per CG iteration",
         "n_gpus": 1,
         "steps": args.steps,
         "warmup": args.warmup,
-        "ms_per_step": ms_per_step,
+        "ms_per_step": op["ms_per_step"],
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
@@ -481,7 +522,8 @@ def main():
                                 f"{cfg.ndet} det x {cfg.nseg * cfg.ns} samples, NSIDE {cfg.nside}, "
                                 f"segments of {cfg.ns}, FP64 block-Jacobi PCG"),
                    "nside": cfg.nside, "ndet": cfg.ndet, "samples": ntot,
-                   "segment": sorted(set(lens)) if uneven else cfg.ns, "npix": npix, "precond": "block",
+                   "segment": sorted(set(cfg.seglen)) if uneven else cfg.ns, "npix": head["npix"],
+                   "precond": "block",
                    "deflate": False, "precision": "fp64", "residual_refresh_every": 10},
         "time_to_1e-6_s": tts,
         "iterations_to_1e-6": head["iterations"] if head["converged"] else None,
@@ -489,18 +531,15 @@ def main():
         "setup_s": head["upload_s"] + head["pixelize_s"] + head["setup_s"] + head["begin_s"],
         "phases_s": {k: head[k] for k in ("upload_s", "pixelize_s", "setup_s", "begin_s")},
         "idle_before_each_pipeline_s": args.settle,
-        "operator_ms": apply_ms,
-        "operator_alg_bytes": b_alg(8),
-        "operator_frac_hbm": b_alg(8) / (apply_ms * 1e-3) / HBM_PEAK,
+        "operator_ms": op["operator_ms"],
+        "operator_alg_bytes": op["operator_alg_bytes"],
+        "operator_frac_hbm": op["operator_frac_hbm"],
         "device_bytes": head["device_bytes"],
-        "run_records": {"records": nrec, "per_sample": rps, "used": runs_on},
-        "streams": {"filtered": nstr, "lines_of_sight": nline, "detectors": cfg.ndet},
+        "run_records": op["run_records"],
+        "streams": op["streams"],
         "fp64_angle_bytes": head["fp64_angle_bytes"],
         "fp64_sorted_angle_bytes": head["fp64_sorted_angle_bytes"],
-        "roofline": {"bound": "hbm", "kernel": names[dom], "achieved": achieved / 1e9,
-                     "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": achieved / HBM_PEAK,
-                     "traffic": traffic, "traffic_source": traffic_src, "bytes_per_launch": alg,
-                     "ms_per_launch": avg_ms, "launches_per_operator": cnt_launch // n_ops},
+        "roofline": op["roofline"],
         "reference_map": {"solver": "the FP64 solve continued to |r|^2/|b|^2 <= 1e-24",
                           "iterations": head["ref_iterations"], "true_residual": head["ref_true_residual"]},
         "map_error_at_1e-6": map_errors(head["map"], ref_map, cnt),
@@ -546,6 +585,23 @@ def main():
             sub["training"]["source"] = ("the weights file's own record, written by the offline run of "
                                          "sanepic_amd.train_precond that made it; no training runs here")
         out[key] = sub
+    if shared:
+        r = shared["fp64"]
+        sub = dict(operator_figures(r, cfg, ntot, args.workload, "fp64-shared"),
+                   operator="detectors that share a line of sight as three streams, mixed bin by bin",
+                   device_bytes=r["device_bytes"])
+        for key, r in shared.items():
+            line = {"time_to_1e-6_s": r["time_to_solution_s"],
+                    "iterations_to_1e-6": r["iterations"] if r["converged"] else None,
+                    "final_true_residual": r["final_true_residual"],
+                    "ms_per_iteration_in_solve": r["solve_s"] * 1e3 / max(r["iterations"], 1),
+                    "setup_s": r["upload_s"] + r["pixelize_s"] + r["setup_s"] + r["begin_s"],
+                    "map_error_vs_fp64_reference": map_errors(r["map"], ref_map, cnt)}
+            if key == "fp64":
+                sub.update(line)
+            else:
+                sub[key] = line
+        out["shared_line_of_sight"] = sub
     if not args.no_cpu:
         try:
             time.sleep(args.settle)

@@ -331,7 +331,8 @@ int sanepic_run_records(sanepic_ctx *ctx, int64_t *nrec, int32_t *active);
  * *lines lines of sight.  Four or more detectors with the same focal-plane
  * offsets are three streams behind one line of sight, mixed bin by bin with
  * their noise weights; otherwise each detector is a stream and a line of its
- * own (both counts are then ndet). */
+ * own (both counts are then ndet).  SANEPIC_STREAMS=0 at creation keeps one
+ * stream per detector. */
 int sanepic_streams(sanepic_ctx *ctx, int32_t *streams, int32_t *lines);
 /* Bytes per sample of the FP64 operator's polarisation angle in its gather
  * and record passes (no counterpart in the reference, which recomputes

@@ -736,6 +736,7 @@ int create_context(const sanepic_config *cfg, sanepic_ctx **out, bool pointing) 
   if (const char *e = getenv("SANEPIC_XCD_BLOCKS")) c->xcd_blocks = atoi(e) != 0;
   if (const char *e = getenv("SANEPIC_ZSORT")) c->zsorted = atoi(e) != 0;
   if (const char *e = getenv("SANEPIC_RUNS")) c->runs = atoi(e) != 0;
+  if (const char *e = getenv("SANEPIC_STREAMS")) c->share = atoi(e) != 0;
   if (const char *e = getenv("SANEPIC_PT_XCD")) c->pt_xcd = atoi(e) != 0;
   if (const char *e = getenv("SANEPIC_MONO_FFT")) c->mono_fft = atoi(e) != 0;
   if (const char *e = getenv("SANEPIC_TURN64")) c->turn64 = atoi(e) != 0;

@@ -47,7 +47,7 @@ bool use_streams(const sanepic_ctx *c) {
 // four streams for every five detectors (16 + 48: 1141 and 1082; 10 + 25: 526
 // and 530).
 int find_streams(sanepic_ctx *c) {
-  if (!c->runs || c->pin_owner || !c->sub.empty() || c->single || c->zsorted || c->nc != 3 || c->g.M != 1 ||
+  if (!c->share || !c->runs || c->pin_owner || !c->sub.empty() || c->single || c->zsorted || c->nc != 3 || c->g.M != 1 ||
       c->pregather || c->recal || c->chunk != 0 || !c->ang64 || c->ndet < 4 || c->ndet > 65535 || c->ns % 16 != 0 ||
       c->cfg.hwp)
     return 0;

@@ -263,6 +263,7 @@ struct sanepic_ctx {
   float *rec32 = nullptr;            // the same of the FP32 operator
   // Detectors that share a line of sight (capi_streams.hip): nstream streams
   // over nline lines of sight, the first nset of them sets of three streams
+  bool share = true;                 // SANEPIC_STREAMS=0: one stream per detector
   int nstream = 0, nset = 0, nline = 0;
   int64_t nsdet = 0;
   SkyStream *d_streams = nullptr;    // [nstream]
