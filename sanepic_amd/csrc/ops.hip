@@ -320,10 +320,12 @@ __device__ __forceinline__ void run_record(const OpArgs<T> &a, uint64_t meta, in
 }
 
 // Columns of P <= 256: the M sub-FFTs side by side.  Thread group j of M (one
-// wave, or two from P = 128 on, which keeps B >= 8 columns a row) transforms
-// the j-th sub-columns of B = 16 G / P columns, the 16 M G values pass through
-// the LDS (FP64: real parts, then imaginary parts), and every thread then makes
-// the radix-M DFT of up to 6 (M = 3) or 4 (M = 5) outputs v.  The kernels above
+// wave, or two from P = 128 on: 16 columns a row there instead of 8, 8 instead
+// of 4 at 256; 6 detectors x 6 x 3 * 2^19 samples 1206 us an iteration, 1247
+// with one wave at 128, mixed 744 and 819) transforms the j-th sub-columns of
+// B = 16 G / P columns, the 16 M G values pass through the LDS (FP64: real
+// parts, then imaginary parts; up to 87 KB), and every thread then makes the
+// radix-M DFT of up to 6 (M = 3) or 4 (M = 5) outputs v.  The kernels above
 // run the sub-FFTs one after the other in the same 256 threads and pass their
 // values through the buffer's rows in HBM: bound by latency, since P = 16 makes
 // 256-column blocks, a few dozen of them in small contexts (3 detectors x 5
@@ -418,7 +420,9 @@ __global__ __launch_bounds__((LOG2P <= 6 ? 64 : 128) * M) void k_col_fwd_mw(OpAr
 
 // The inverse: radix-M DFTs first, their values to the sub-FFTs' groups
 // through the LDS whole (80 KB for M = 5 in FP64; in two halves the outputs
-// waiting in registers took 256 of them), then a wave per sub-FFT.
+// waiting in registers took 256 of them), then a wave per sub-FFT.  From P = 32
+// on a CU holds one such block of five waves: not for its LDS, but because 170
+// registers leave room for two waves a SIMD, eight a CU.
 template <typename T, int LOG2P, int M>
 __global__ __launch_bounds__(64 * M) void k_col_inv_mw(OpArgs<T> a) {
   using V = VT<T>;
