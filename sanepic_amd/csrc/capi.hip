@@ -146,6 +146,14 @@ int build_tables(sanepic_ctx *c) {
 int build_weights(sanepic_ctx *c) {
   if (c->wt) return 0;
   const int64_t N = c->ns, H = N / 2 + 1;
+  if (use_streams(c)) {
+    int rc = dalloc(c, c->mix, 6 * (int64_t)c->nset * N);
+    if (!rc && c->cfg.precision == SANEPIC_MIXED) rc = dalloc(c, c->mix32, 6 * (int64_t)c->nset * N);
+    if (rc) {  // no room for them: one stream per detector
+      ACHK(c, drop_streams(c));
+      ACHK(c, sorted_turns(c));
+    }
+  }
   // the half spectra go up; the row-layout transposition runs on the device
   double *dspn = nullptr;
   ACHK(c, dalloc(c, dspn, c->ndet * H));
@@ -154,11 +162,8 @@ int build_weights(sanepic_ctx *c) {
   ACHK(c, dalloc(c, c->wt, c->ndet * N));
   if (c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->wt32, c->ndet * N));
   LCHK(c, launch_build_weights(dspn, c->ndet, N, c->g.N1, c->g.N2, c->wt, c->wt32, c->st));
-  if (use_streams(c)) {
-    ACHK(c, dalloc(c, c->mix, 6 * (int64_t)c->nset * N));
-    if (c->cfg.precision == SANEPIC_MIXED) ACHK(c, dalloc(c, c->mix32, 6 * (int64_t)c->nset * N));
+  if (use_streams(c))
     LCHK(c, launch_build_mix(dspn, c->d_sdet, c->d_sbeg, c->nset, N, c->g.N1, c->g.N2, c->mix, c->mix32, c->st));
-  }
   HIPCHK(c, hipStreamSynchronize(c->st));
   dfree_later(c, dspn, c->ndet * H);
   return 0;

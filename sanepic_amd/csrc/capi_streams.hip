@@ -27,6 +27,16 @@ bool use_streams(const sanepic_ctx *c) {
   return c->nstream > 0 && use_runs(c);
 }
 
+static void free_streams(sanepic_ctx *c) {
+  dfree(c, c->line_pix, (int64_t)c->nline * c->nseg * c->ns);
+  dfree(c, c->d_streams, c->nstream);
+  dfree(c, c->d_sdet, c->nsdet);
+  dfree(c, c->d_sbeg, c->nset + 1);
+  dfree(c, c->mix, 6 * (int64_t)c->nset * c->ns);
+  dfree(c, c->mix32, 6 * (int64_t)c->nset * c->ns);
+  c->nstream = c->nset = c->nline = 0;
+}
+
 // Finds the sets (equal offsets, and the same pixels sample by sample: a
 // sample without pointing takes the pixel before it, which may be another
 // detector's) at pixelisation, while c->pix holds compressed pixels.  Only
@@ -109,14 +119,15 @@ int find_streams(sanepic_ctx *c) {
   c->nset = nset;
   c->nline = line;
   c->nsdet = (int64_t)sdet.size();
-  ACHK(c, dalloc(c, c->d_streams, c->nstream));
-  ACHK(c, dalloc(c, c->d_sdet, c->nsdet));
-  ACHK(c, dalloc(c, c->d_sbeg, nset + 1));
+  // line_pix: the lines' pixels [nline][nseg ns], from which the run layout is built
+  if (dalloc(c, c->d_streams, c->nstream) || dalloc(c, c->d_sdet, c->nsdet) || dalloc(c, c->d_sbeg, nset + 1) ||
+      dalloc(c, c->line_pix, (int64_t)line * c->nseg * c->ns)) {
+    free_streams(c);  // no room for them: one stream per detector
+    return 0;
+  }
   HIPCHK(c, hipMemcpy(c->d_streams, vs.data(), vs.size() * sizeof(SkyStream), hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(c->d_sdet, sdet.data(), sdet.size() * sizeof(SkyDet), hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(c->d_sbeg, sbeg.data(), sbeg.size() * 4, hipMemcpyHostToDevice));
-  // the lines' pixels [nline][nseg ns], from which the run layout is built
-  ACHK(c, dalloc(c, c->line_pix, (int64_t)line * c->nseg * c->ns));
   std::vector<int32_t> first((size_t)line);
   for (const SkyStream &v : vs) first[(size_t)v.set] = v.det;
   const int64_t spd = c->nseg * c->ns;
@@ -125,18 +136,13 @@ int find_streams(sanepic_ctx *c) {
   return 0;
 }
 
-// Back to one stream per detector (relative calibration chosen after the
-// pixelisation: its gains differ between the detectors of a set).
+// Back to one stream per detector: relative calibration chosen after the
+// pixelisation (its gains differ between the detectors of a set), or no room for
+// the mixing weights.
 int drop_streams(sanepic_ctx *c) {
   if (!c->nstream) return 0;
   HIPCHK(c, hipStreamSynchronize(c->st));
   const int64_t nl = (int64_t)c->nline * c->nseg * c->ns;
-  dfree(c, c->line_pix, nl);
-  dfree(c, c->d_streams, c->nstream);
-  dfree(c, c->d_sdet, c->nsdet);
-  dfree(c, c->d_sbeg, c->nset + 1);
-  dfree(c, c->mix, 6 * (int64_t)c->nset * c->ns);
-  dfree(c, c->mix32, 6 * (int64_t)c->nset * c->ns);
   dfree(c, c->rmeta, nl / 16);
   dfree(c, c->rperm, c->nrec);
   dfree(c, c->rec64, 5 * c->nrec);
@@ -151,8 +157,8 @@ int drop_streams(sanepic_ctx *c) {
   dfree(c, r.sp_count, r.items.nsplit);
   dfree(c, r.partial, 8 * std::max<int64_t>(1, r.nslots));
   c->ritems = ItemSet();
-  c->nstream = c->nset = c->nline = 0;
   c->nrec = 0;
+  free_streams(c);
   ACHK(c, build_runs(c));
   return c->split_chosen ? 0 : set_split(c, default_split(c));
 }

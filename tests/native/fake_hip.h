@@ -12,7 +12,8 @@ inline double cospi(double x) { return std::cos(M_PI * x); }  // a device functi
 #include "ctx.h"
 
 namespace fake {
-int64_t room = 0, frees = 0, mallocs = 0;
+int64_t room = 0;
+size_t refuse = 0;  // a request of this size fails
 std::map<void *, int64_t> live;
 char *next = (char *)((uintptr_t)1 << 44);
 inline int64_t held() {
@@ -32,9 +33,8 @@ inline int64_t held() {
 
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) {
-  if ((int64_t)n > fake::room) return hipErrorOutOfMemory;
+  if ((int64_t)n > fake::room || n == fake::refuse) return hipErrorOutOfMemory;
   fake::room -= (int64_t)n;
-  fake::mallocs++;
   *p = fake::next;
   fake::live[*p] = (int64_t)n;
   fake::next += (n + 4095) / 4096 * 4096 + 4096;
@@ -47,11 +47,17 @@ hipError_t hipFree(void *p) {
     std::exit(1);
   }
   fake::room += b->second;
-  fake::frees++;
   fake::live.erase(b);
   return hipSuccess;
 }
 hipError_t hipMemcpy(void *, const void *, size_t, hipMemcpyKind) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void *, const void *, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  *p = std::calloc(n, 1);
+  return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipMemGetInfo(size_t *f, size_t *t) {

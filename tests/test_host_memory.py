@@ -13,7 +13,7 @@ NATIVE = os.path.join(ROOT, "tests", "native")
 LIBDIR = os.path.dirname(sanepic_amd.LIB_PATH)
 
 
-@pytest.mark.parametrize("program", ["recal_state", "arena_state"])
+@pytest.mark.parametrize("program", ["recal_state", "arena_state", "streams_memory"])
 def test_native(program, tmp_path):
     exe = str(tmp_path / program)
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
