@@ -293,8 +293,12 @@ int group_pixelize(sanepic_ctx *c, int64_t *npix_out, int64_t *ndef_out) {
 // for each other; on four queues (the hardware's) the passes of different
 // groups fill it: an application to 12 detectors of 2^21 samples in nine groups
 // took 980 us on one queue, 710 us on four.  Longest group first, to the queue
-// with the fewest samples (counting odd radices 1.5 times changes nothing: 570
-// and 572 us, 734 and 738 at 8 detectors of 2^22).
+// with the least work; a sample of an odd radix counts 1.5 times, since its
+// columns' passes take longer: the first group's queue is the context's stream,
+// which P^T follows without a wait for another queue (16 iterations over 128
+// segments of 2^14, 3 of 5 x 2^17 and 1 of 5 x 2^18: 4.93 ms with the radix-5
+// group of 3 there, 5.09 with the longer one of 2^14; 570 and 572 us an
+// application with the 12 detectors above).
 int make_queues(sanepic_ctx *c) {
   const size_t ng = c->sub.size();
   if (!c->union_pt || ng < 2 || !c->gqueue.empty()) return 0;
@@ -305,7 +309,7 @@ int make_queues(sanepic_ctx *c) {
   }
   std::vector<size_t> order(ng);
   std::iota(order.begin(), order.end(), (size_t)0);
-  auto work = [&](size_t k) { return (double)c->sub[k]->ntot; };
+  auto work = [&](size_t k) { return (double)c->sub[k]->ntot * (c->sub[k]->g.M > 1 ? 1.5 : 1.0); };
   std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return work(a) > work(b); });
   double load[sanepic_ctx::kQueues] = {0.0};
   c->gqueue.assign(ng, 0);

@@ -376,13 +376,21 @@ inline Arena &arena_of(sanepic_ctx *c) { return c->pin_owner ? c->pin_owner->are
 // size: the groups' temporaries, released one group after the other, serve the
 // next group, and a release of even the smallest to the runtime would wait for
 // the TOD uploads in flight (64 detectors x 2^24 samples: 0.12 s in the first
-// group's pixelisation).  Larger ones take a spare block if one fits, such as
-// the groups' temporaries during the parent's pixelisation, else the device.
+// group's pixelisation).  Larger ones come from the device; the parent of groups
+// takes a spare block first if one fits, such as the groups' temporaries during
+// its pixelisation, every context where the device has no more.
 constexpr int64_t kArenaMin = int64_t(1) << 20, kArenaMax = int64_t(1) << 27;
 
 inline hipError_t dev_alloc(sanepic_ctx *c, void **v, int64_t bytes) {
   if (!c->pin_owner && bytes < kArenaMin) return hipMalloc(v, (size_t)bytes);
   Arena &a = arena_of(c);
+  if (!c->pin_owner && bytes >= kArenaMax && c->sub.empty()) {
+    const hipError_t e = hipMalloc(v, (size_t)bytes);
+    if (e == hipSuccess) return e;
+    *v = a.take(bytes);
+    if (*v) (void)hipGetLastError();
+    return *v ? hipSuccess : e;
+  }
   *v = a.take(bytes);
   if (*v) return hipSuccess;
   if (!c->pin_owner && bytes >= kArenaMax) return hipMalloc(v, (size_t)bytes);
