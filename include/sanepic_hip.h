@@ -182,8 +182,9 @@ int sanepic_get_indpix(sanepic_ctx *ctx, int64_t *indpix);
  * sanepic_autotune times one operator application for every admissible
  * split on the context's own pointing and keeps the fastest; with a cache
  * path the choice is looked up in (and appended to) that text file, keyed
- * by device architecture, sizes and precision.  Both calls belong between
- * sanepic_pixelize and sanepic_setup.  log2_n1 / op_ms may be NULL. */
+ * by device architecture, sizes, precision and the passes the context runs.
+ * Both calls belong between sanepic_pixelize and sanepic_setup.  log2_n1 /
+ * op_ms may be NULL. */
 int sanepic_autotune(sanepic_ctx *ctx, const char *cache, int32_t *log2_n1,
                      double *op_ms);
 int sanepic_set_fft_split(sanepic_ctx *ctx, int32_t log2_n1);
